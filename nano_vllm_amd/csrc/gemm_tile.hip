@@ -15,6 +15,7 @@
 // Requires K % 64 == 0 and 16-byte aligned rows; the launcher refuses anything else (code 1) and the
 // caller runs another kernel.
 #include "common.h"
+#include "lds_load.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
@@ -40,12 +41,6 @@ struct TileArgs {
     int cols_per_wg;        // columns of y a workgroup takes: those of its tile, or fewer (the tile's other rows of W are not fetched)
 };
 
-// 16 bytes per lane from base + offset (base the same for the whole wave, offset in bytes per lane)
-// to LDS at lds + 16 * lane (lds the same for the whole wave).  Written by hand: the compiler would
-// make every later read of LDS wait for all such loads; these are waited for by count.
-__device__ __forceinline__ void tl_load_to_lds(const __bf16* base, uint32_t offset, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "s"(lds) : "memory", "m0");
-}
 // Workgroups walk the chunks of their range in rotated order, each from another start: at one k the
 // rows of a tile (a power of two apart, as a rule) lie in few channels of the memory and of the L2,
 // and workgroups that all fetch the same k at the same time queue up there.  (Past the range's end:
@@ -54,10 +49,6 @@ __device__ __forceinline__ uint32_t tl_chunk_offset(int c, int chunks, int rot) 
     const int cc = min(c, chunks - 1) + rot;
     return (uint32_t)(cc >= chunks ? cc - chunks : cc) * TL_ROW_BYTES;
 }
-// (the counter of loads on their way has six bits: the launcher refuses what would need more)
-template <int N> __device__ __forceinline__ void tl_wait_loads_but() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N < 64 ? N : 63) : "memory"); }
-__device__ __forceinline__ void tl_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
 // The products of one chunk of 64 k: x_stage and w_stage are the chunk's tiles in LDS, a_row / b_row
 // the byte offsets of this lane's row in the first 32-row block of its wave's part, slot[ks] the byte
 // offset of its piece in k step ks.  The fragments of a step are read while the products of the step
@@ -190,7 +181,7 @@ linear_tile_kernel(const TileArgs a) {
         const uint32_t k_off = tl_chunk_offset(c, chunks, rot);
 #pragma unroll
         for (int i = 0; i < LOADS; ++i)
-            tl_load_to_lds(i < X_LOADS ? a.x : a.w, src[i] + k_off, __builtin_amdgcn_readfirstlane(stage + i * TL_WAVES * 1024));
+            nva_load_to_lds(i < X_LOADS ? a.x : a.w, src[i] + k_off, __builtin_amdgcn_readfirstlane(stage + i * TL_WAVES * 1024));
     };
 
     // ---- what this lane reads: row lane % 32 of each 32-row block of its wave's part, pieces 2 * ks + lane / 32
@@ -213,13 +204,13 @@ linear_tile_kernel(const TileArgs a) {
 #pragma unroll
     for (int s = 0; s < STAGES - 1; ++s) issue(s);
     for (int c = 0; c < chunks; ++c) {
-        tl_wait_loads_but<LOADS * (STAGES - 2)>();                // this wave's part of chunk c has landed
-        tl_barrier();                                             // everybody's has, and chunk c - 1 is done with
+        nva_wait_loads_but<LOADS * (STAGES - 2)>();                // this wave's part of chunk c has landed
+        nva_lds_barrier();                                             // everybody's has, and chunk c - 1 is done with
         issue(c + STAGES - 1);
         const char* stage = tl_lds + (c % STAGES) * STAGE_BYTES;
         tile_chunk<TM, TN>(stage, stage, a_row, b_row, slot, acc);
     }
-    tl_wait_loads_but<0>();                                       // the loads past the end, before the workgroup leaves
+    nva_wait_loads_but<0>();                                       // the loads past the end, before the workgroup leaves
     tile_store<TM, TN, BN / WN>(a, acc, m0 + wm * (BM / WM), n0, wn, lane);
 }
 
@@ -257,16 +248,16 @@ linear_tile_fed_kernel(const TileArgs a) {
             const uint32_t stage = lds_base + (uint32_t)(c % SX) * X_STAGE;
             const uint32_t k_off = tl_chunk_offset(c, chunks, rot);
 #pragma unroll
-            for (int i = 0; i < XL; ++i) tl_load_to_lds(a.x, src[i] + k_off, __builtin_amdgcn_readfirstlane(stage + i * 1024));
+            for (int i = 0; i < XL; ++i) nva_load_to_lds(a.x, src[i] + k_off, __builtin_amdgcn_readfirstlane(stage + i * 1024));
         };
 #pragma unroll
         for (int s = 0; s < SX - 1; ++s) issue(s);
         for (int c = 0; c < chunks; ++c) {
-            tl_wait_loads_but<XL * (SX - 2)>();
-            tl_barrier();
+            nva_wait_loads_but<XL * (SX - 2)>();
+            nva_lds_barrier();
             issue(c + SX - 1);
         }
-        tl_wait_loads_but<0>();
+        nva_wait_loads_but<0>();
         return;
     }
     // ---- the waves that multiply; load i of wave w fills rows 8 * (4 i + w) .. + 7 of a W tile
@@ -281,7 +272,7 @@ linear_tile_fed_kernel(const TileArgs a) {
         const uint32_t stage = lds_base + SX * X_STAGE + (uint32_t)(c % SW) * W_STAGE + wave * 1024;
         const uint32_t k_off = tl_chunk_offset(c, chunks, rot);
 #pragma unroll
-        for (int i = 0; i < WL; ++i) tl_load_to_lds(a.w, src[i] + k_off, __builtin_amdgcn_readfirstlane(stage + i * TL_WAVES * 1024));
+        for (int i = 0; i < WL; ++i) nva_load_to_lds(a.w, src[i] + k_off, __builtin_amdgcn_readfirstlane(stage + i * TL_WAVES * 1024));
     };
     const int wm = wave / WN, wn = wave % WN;
     const int half = lane / 32, r32 = lane % 32;
@@ -301,12 +292,12 @@ linear_tile_fed_kernel(const TileArgs a) {
 #pragma unroll
     for (int s = 0; s < SW - 1; ++s) issue(s);
     for (int c = 0; c < chunks; ++c) {
-        tl_wait_loads_but<WL * (SW - 2)>();                       // this wave's part of W chunk c has landed
-        tl_barrier();                                             // all of chunk c has, and chunk c - 1 is done with
+        nva_wait_loads_but<WL * (SW - 2)>();                       // this wave's part of W chunk c has landed
+        nva_lds_barrier();                                             // all of chunk c has, and chunk c - 1 is done with
         issue(c + SW - 1);
         tile_chunk<TM, TN>(tl_lds + (c % SX) * X_STAGE, tl_lds + SX * X_STAGE + (c % SW) * W_STAGE, a_row, b_row, slot, acc);
     }
-    tl_wait_loads_but<0>();
+    nva_wait_loads_but<0>();
     tile_store<TM, TN, BN / WN>(a, acc, m0 + wm * (BM / WM), n0, wn, lane);
 }
 

@@ -30,6 +30,7 @@
 // what else is in the batch or on where its row fell among the sorted ones; operands and results are elements
 // (rounded once), the combination is float.
 #include "common.h"
+#include "lds_load.h"
 
 #define MOE_BM 32
 #define MOE_BN 64
@@ -161,11 +162,13 @@ moe_plan_kernel(const int32_t* __restrict__ ids, int64_t pairs, int experts, int
     }
     __syncthreads();
     for (int e = threadIdx.x; e < experts; e += blockDim.x) {
-        const int n = count_s[e];
-        for (int i = 0; i * bm < n; ++i) {
+        // an expert's rows in as few tiles as hold them, shared out evenly over these (a tile's products are made
+        // for whole blocks of 16 rows, so even tiles leave fewer empty rows than full ones and a rest)
+        const int n = count_s[e], parts = (n + bm - 1) / bm, per = parts ? (n + parts - 1) / parts : 0;
+        for (int i = 0; i < parts; ++i) {
             tile_expert[tile0_s[e] + i] = e;
-            tile_row0[tile0_s[e] + i] = begin_s[e] + i * bm;
-            tile_rows[tile0_s[e] + i] = min(bm, n - i * bm);
+            tile_row0[tile0_s[e] + i] = begin_s[e] + i * per;
+            tile_rows[tile0_s[e] + i] = min(per, n - i * per);
         }
     }
     for (int64_t i = threadIdx.x; i < pairs; i += blockDim.x) {
@@ -255,6 +258,9 @@ moe_tile_kernel(const T* __restrict__ a, int64_t a_stride, const T* __restrict__
 typedef __attribute__((ext_vector_type(8))) __bf16 moe_bf16x8;
 typedef __attribute__((ext_vector_type(4))) float moe_f32x4;
 #define MOE_KC 128
+#define MW_ROWS 256              // rows of a tile of the kernel for experts of many rows, at most
+// ... and the rows an expert from which it is the faster one, with a gate and without (moe_tile_rows)
+#define MW_MIN(gated) ((gated) ? 16 : 28)
 
 template <int BM, int WR, bool UP, bool GATED = false>
 __global__ void __launch_bounds__(256)
@@ -362,6 +368,140 @@ moe_mfma_kernel(const __bf16* __restrict__ a, int64_t a_stride, const __bf16* __
             }
         }
 }
+
+// ---------------------------------------------------------------------------- tiles of many rows
+// The same products for experts of many rows: a workgroup of eight waves takes up to 256 rows and 256 rows of the expert's
+// matrix (256 outputs; gated: 128 outputs, their gate rows and their up rows), and both go from global memory straight
+// into LDS, 64 columns a stage, two stages in turn.  A wave multiplies half the tile's rows with 64 rows of the matrix,
+// 16 rows by 16 as the small tiles do (the same sums in the same order, so the same bits whichever kernel took a row).
+// Bound by what the L2s give the CUs: a stage of 64 KB feeds 8.4 MFLOP, 0.93 PFLOP/s are 7.3 TB/s.  The larger the tile
+// the fewer bytes a product needs: tiles of 128 rows ran at 0.75 PFLOP/s (4096 tokens, 8 of 32 experts of 4096 x 1536).
+// The products of 2048 tokens, 8 of 30 gated experts of 2048 x 768, plan and sum included: 491 us with the matrix going
+// from global memory into the waves' registers, 234 here; 6 of 32 without a gate 294 and 143.  An expert's rows are shared
+// out evenly over its tiles, and a wave multiplies as many blocks of 16 rows as its tile has (292 us with whole tiles).
+typedef __attribute__((ext_vector_type(4))) __bf16 moe_bf16x4;
+struct MoeWideArgs {
+    const __bf16* a; int64_t a_stride; const __bf16* w; int n, k;
+    const int32_t* rows; int top;
+    const int32_t* tile_expert; const int32_t* tile_row0; const int32_t* tile_rows; const int32_t* num_tiles;
+    int col_tiles, act; __bf16* out; int64_t out_stride;
+};
+
+// MB: blocks of 16 rows of a wave's half of the tile.
+template <int MB, bool UP, bool GATED>
+__device__ __forceinline__ void moe_wide_tile(const MoeWideArgs& p, int e, int row0, int nrows, int n0) {
+    constexpr int WAVES = 8, ROW_BYTES = 128, LOAD_ROWS = 8;               // rows of a stage that one load of a wave fills
+    constexpr int X_LOADS = (MB + 1) / 2, W_LOADS = 4, LOADS = X_LOADS + W_LOADS;
+    constexpr int STAGE_BYTES = (MW_ROWS + 256) * ROW_BYTES, X_BYTES = MW_ROWS * ROW_BYTES;
+    extern __shared__ __attribute__((aligned(1024))) char mw_lds[];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / NVA_WAVE), lane = threadIdx.x % NVA_WAVE;
+    const int wm = wave / 4, wn = wave % 4, col = lane & 15, g = lane >> 4;
+    const int n = p.n, k = p.k;
+    const __bf16* we = p.w + (int64_t)e * (GATED ? 2 : 1) * n * k;
+    // what this lane fetches: 16 bytes of a row; which piece of a row lies where is turned with the row's number, so
+    // that the 16 rows of a read lie in different banks
+    const int piece = (lane % 8) ^ ((lane / 16 + 4 * (wave & 1)) % 8);     // (row / 2) % 8 of row 8 (8 i + wave) + lane / 8
+    uint32_t src[LOADS];
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+        const int r = LOAD_ROWS * ((i < X_LOADS ? i : i - X_LOADS) * WAVES + wave) + lane / 8;
+        int64_t at;
+        if (i < X_LOADS) {
+            const int q = min(r, nrows - 1);
+            at = (int64_t)(UP ? p.rows[row0 + q] / p.top : row0 + q) * p.a_stride;
+        } else {
+            at = GATED ? ((int64_t)min(n0 + r / 64 * 32 + r % 32, n - 1) + (r % 64 < 32 ? 0 : n)) * k : (int64_t)min(n0 + r, n - 1) * k;
+        }
+        src[i] = (uint32_t)((at + piece * 8) * 2);
+    }
+    const uint32_t lds_base = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)mw_lds + wave * 1024;
+    const int chunks = k / 64;
+    auto issue = [&](int c) __attribute__((always_inline)) {               // (past the end: the last chunk again)
+        const uint32_t stage = lds_base + (uint32_t)(c & 1) * STAGE_BYTES;
+        const uint32_t k_off = (uint32_t)min(c, chunks - 1) * ROW_BYTES;
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i)
+            nva_load_to_lds(i < X_LOADS ? p.a : we, src[i] + k_off,
+                            __builtin_amdgcn_readfirstlane(stage + (i < X_LOADS ? i * 8192 : X_BYTES + (i - X_LOADS) * 8192)));
+    };
+    const uint32_t x_row = (uint32_t)(wm * MB * 16 + col) * ROW_BYTES, w_row = X_BYTES + (uint32_t)(wn * 64 + col) * ROW_BYTES;
+    const uint32_t turn_w = (uint32_t)(col / 2), turn_x = (uint32_t)((wm * MB * 16 + col) / 2 % 8);
+    moe_f32x4 acc[4][MB];
+#pragma unroll
+    for (int f = 0; f < 4; ++f)
+#pragma unroll
+        for (int b = 0; b < MB; ++b) acc[f][b] = moe_f32x4{0.f, 0.f, 0.f, 0.f};
+    issue(0);
+    for (int c = 0; c < chunks; ++c) {
+        nva_wait_loads_but<0>();
+        nva_lds_barrier();
+        issue(c + 1);
+        const char* stage = mw_lds + (c & 1) * STAGE_BYTES;
+        moe_bf16x8 fw[2][4], fx[2][MB];
+        auto read = [&](int ks) __attribute__((always_inline)) {
+#pragma unroll
+            for (int f = 0; f < 4; ++f) fw[ks][f] = *reinterpret_cast<const moe_bf16x8*>(stage + w_row + f * 16 * ROW_BYTES + ((4 * ks + g) ^ turn_w) * 16);
+#pragma unroll
+            for (int b = 0; b < MB; ++b) fx[ks][b] = *reinterpret_cast<const moe_bf16x8*>(stage + x_row + b * 16 * ROW_BYTES + ((4 * ks + g) ^ turn_x) * 16);
+        };
+        auto multiply = [&](int ks) __attribute__((always_inline)) {
+#pragma unroll
+            for (int b = 0; b < MB; ++b)
+#pragma unroll
+                for (int f = 0; f < 4; ++f) acc[f][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[ks][f], fx[ks][b], acc[f][b], 0, 0, 0);
+        };
+        // the second half of the stage is read between the products of the first
+        read(0);
+        __builtin_amdgcn_sched_barrier(0);
+        read(1);
+        multiply(0);
+#pragma unroll
+        for (int i = 0; i < 4 + MB; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);             // one read of LDS,
+            __builtin_amdgcn_sched_group_barrier(0x008, 4 * MB / (4 + MB), 0);   // and as many products as there are for it
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(1);
+    }
+    nva_wait_loads_but<0>();
+    // acc[f][b][i] = out[row 16 b + col][16 f + 4 g + i of the wave's 64] (gated: fragments 2 and 3 hold the up sums)
+#pragma unroll
+    for (int b = 0; b < MB; ++b) {
+        const int r = wm * MB * 16 + 16 * b + col;
+        if (r >= nrows) continue;
+        __bf16* o = p.out + (int64_t)(row0 + r) * p.out_stride;
+#pragma unroll
+        for (int f = 0; f < (GATED ? 2 : 4); ++f) {
+            const int c = n0 + wn * (GATED ? 32 : 64) + 16 * f + 4 * g;
+            moe_bf16x4 v;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float y = acc[f][b][i];
+                if (GATED) y = nva_gate_act(p.act, y) * acc[GATED ? f + 2 : f][b][i];
+                else if (UP) y = nva_gate_act(p.act, y);
+                v[i] = (__bf16)y;
+            }
+            if (c < n) *reinterpret_cast<moe_bf16x4*>(o + c) = v;          // n is a multiple of 4
+        }
+    }
+}
+
+template <bool UP, bool GATED>
+__global__ void __launch_bounds__(512)
+moe_wide_kernel(const MoeWideArgs p) {
+    // a run of neighbouring tiles on every die: tiles of one expert share its matrix, those of one row tile its rows
+    const int total = p.num_tiles[0] * p.col_tiles, per = (total + NVA_XCDS - 1) / NVA_XCDS;
+    const int j = (int)(blockIdx.x / NVA_XCDS), unit = (int)(blockIdx.x % NVA_XCDS) * per + j;
+    if (j >= per || unit >= total) return;
+    const int tile = unit / p.col_tiles, n0 = unit % p.col_tiles * (GATED ? 128 : 256);
+    const int e = p.tile_expert[tile], row0 = p.tile_row0[tile], nrows = p.tile_rows[tile];
+    // half the rows in blocks of 16, rounded up to an even number of blocks
+    const int mb = (nrows + 63) / 64;
+    if (mb == 4) moe_wide_tile<8, UP, GATED>(p, e, row0, nrows, n0);
+    else if (mb == 3) moe_wide_tile<6, UP, GATED>(p, e, row0, nrows, n0);
+    else if (mb == 2) moe_wide_tile<4, UP, GATED>(p, e, row0, nrows, n0);
+    else moe_wide_tile<2, UP, GATED>(p, e, row0, nrows, n0);
+}
 #endif
 
 template <typename T>
@@ -433,15 +573,28 @@ NVA_EXPORT int NVA_NAME(nva_moe_route)(const float* logits, int64_t stride, int6
     return nva_check_launch("moe_route");
 }
 
-// Rows of a tile of the experts' products for this many pairs (token, choice) and experts: the plan's arrays are
-// sized with it.  Many rows an expert: tall tiles, so that an expert's matrix is read few times.
-static int moe_tile_rows(int64_t pairs, int experts, int k, int ff) {
+// Rows of a tile of the experts' products: the plan's arrays are sized with it.  From MW_MIN rows an expert on (on
+// average) the kernel for many rows takes them; a tile's matrix and rows must lie within 4 GB of each other, since its
+// lanes hold 32-bit offsets.
+// Where the line lies (the whole call, 32 experts of 2048 x 768, in us, 32-row tiles / this kernel): gated 8 rows an expert
+// 75 / 73, 16 rows 87 / 80, 32 rows 124 / 77; without a gate 12 rows 50 / 54, 24 rows 50 / 56, 32 rows
+// 80 / 57.  Sizes that are no multiple of 64 keep the tiles of 32 and 128 rows.
+static int moe_tile_rows(const void* x, int64_t x_stride, const void* up, const void* down, int64_t tokens, int top, int experts,
+                         int k, int ff, int gated) {
 #if defined(NVA_BF16)
-    if (k % 8 == 0 && ff % 8 == 0) return pairs >= 64 * (int64_t)experts ? 128 : 32;
+    const int64_t pairs = tokens * top, most = 1LL << 31;
+    if (k % 8 == 0 && ff % 8 == 0 && x_stride % 8 == 0 && nva_aligned(x, 16) && nva_aligned(up, 16) && nva_aligned(down, 16)) {
+        if (pairs < MW_MIN(gated) * (int64_t)experts) return 32;
+        return k % 64 == 0 && ff % 64 == 0 && tokens * x_stride < most && pairs * ff < most && (int64_t)(gated ? 2 : 1) * ff * k < most
+                   ? MW_ROWS : 128;
+    }
 #endif
     return MOE_BM;
 }
-NVA_EXPORT int NVA_NAME(nva_moe_tile_rows)(int64_t pairs, int experts, int k, int ff) { return moe_tile_rows(pairs, experts, k, ff); }
+NVA_EXPORT int NVA_NAME(nva_moe_tile_rows)(const void* x, int64_t x_stride, const void* up, const void* down, int64_t tokens, int top,
+                                           int experts, int k, int ff, int gated) {
+    return moe_tile_rows(x, x_stride, up, down, tokens, top, experts, k, ff, gated);
+}
 
 // ids from `experts` on are identities (x itself).  add_gate: float, one logit a token gate_stride apart, or null.
 // x [tokens, k] elements; ids, weights [tokens, top]; up [E * ff, k] (gated: [E * 2 ff, k], an expert's gate rows, then
@@ -458,7 +611,7 @@ NVA_EXPORT int NVA_NAME(nva_moe_experts)(const void* x, int64_t x_stride, const 
     const int64_t pairs = tokens * top;
     if (tokens < 0 || top <= 0 || experts <= 0 || experts > MOE_MAX_EXPERTS || k <= 0 || ff <= 0 || pairs > 0x7fffffff)
         return nva_fail("moe_experts: bad sizes tokens=%lld top=%d experts=%d k=%d ff=%d", (long long)tokens, top, experts, k, ff);
-    const int bm = moe_tile_rows(pairs, experts, k, ff);
+    const int bm = moe_tile_rows(x, x_stride, up, down, tokens, top, experts, k, ff, gated);
     if (max_tiles < pairs / bm + experts || max_tiles > 0x7fffffff)
         return nva_fail("moe_experts: room for %lld tiles, %lld may be needed", (long long)max_tiles, (long long)(pairs / bm + experts));
     if (act < 0 || act > 3) return nva_fail("moe_experts: unknown activation %d", act);
@@ -472,8 +625,8 @@ NVA_EXPORT int NVA_NAME(nva_moe_experts)(const void* x, int64_t x_stride, const 
                        tile_row0, tile_rows, num_tiles);
     if ((ff + MOE_BN - 1) / MOE_BN > 65535 || (k + MOE_BN - 1) / MOE_BN > 65535) return nva_fail("moe_experts: too wide");
 #if defined(NVA_BF16)
-    if (k % 8 == 0 && ff % 8 == 0 && x_stride % 8 == 0 && nva_aligned(x, 16) && nva_aligned(up, 16) && nva_aligned(down, 16) &&
-        nva_aligned(hidden, 16)) {
+    if (k % 8 == 0 && ff % 8 == 0 && x_stride % 8 == 0 && nva_aligned(x, 16) && nva_aligned(up, 16) && nva_aligned(down, 16)) {
+        if (!nva_aligned(hidden, 16) || !nva_aligned(outs, 16)) return nva_fail("moe_experts: scratch that is not aligned to 16 bytes");
 #define MOE_LAUNCH(BMV, WRV)                                                                                                  \
         hipLaunchKernelGGL((moe_mfma_kernel<BMV, WRV, true>), dim3((unsigned)max_tiles, (ff + 4 * WRV - 1) / (4 * WRV)),        \
                            dim3(256), 0, stream, (const __bf16*)x, x_stride, (const __bf16*)up, ff, k, rows, top, tile_expert, \
@@ -488,7 +641,22 @@ NVA_EXPORT int NVA_NAME(nva_moe_experts)(const void* x, int64_t x_stride, const 
         hipLaunchKernelGGL((moe_mfma_kernel<BMV, WRV / 2, false>), dim3((unsigned)max_tiles, (k + 2 * WRV - 1) / (2 * WRV)),    \
                            dim3(256), 0, stream, (const __bf16*)hidden, (int64_t)ff, (const __bf16*)down, k, ff, rows, top,     \
                            tile_expert, tile_row0, tile_rows, num_tiles, act, (__bf16*)outs, (int64_t)k)
-        if (gated) {
+        if (bm == MW_ROWS) {
+            const int lds = 2 * (MW_ROWS + 256) * 128;
+#define MOE_LAUNCH_WIDE(UPV, GATEDV, A, AS, W, N, K, CT, O)                                                                    \
+            do {                                                                                                              \
+                const auto kernel = moe_wide_kernel<UPV, GATEDV>;                                                             \
+                if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)  \
+                    return nva_fail("moe_experts: %d bytes of LDS are not to be had", lds);                                   \
+                const MoeWideArgs p = {(const __bf16*)(A), AS, (const __bf16*)(W), N, K, rows, top, tile_expert, tile_row0,   \
+                                       tile_rows, num_tiles, CT, act, (__bf16*)(O), (int64_t)(N)};                            \
+                hipLaunchKernelGGL(kernel, dim3((unsigned)(max_tiles * (CT))), dim3(512), lds, stream, p);                    \
+            } while (0)
+            if (gated) MOE_LAUNCH_WIDE(true, true, x, x_stride, up, ff, k, (ff + 127) / 128, hidden);
+            else MOE_LAUNCH_WIDE(true, false, x, x_stride, up, ff, k, (ff + 255) / 256, hidden);
+            MOE_LAUNCH_WIDE(false, false, hidden, (int64_t)ff, down, k, ff, (k + 255) / 256, outs);
+#undef MOE_LAUNCH_WIDE
+        } else if (gated) {
             if (bm == 128) { MOE_LAUNCH_GATED(128, 64); } else { MOE_LAUNCH_GATED(32, 32); }
         } else if (bm == 128) { MOE_LAUNCH(128, 32); } else { MOE_LAUNCH(32, 16); }
 #undef MOE_LAUNCH_GATED

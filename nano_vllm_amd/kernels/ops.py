@@ -910,7 +910,8 @@ class HipKernels:
             gate_stride = add_gate.stride(0)
         pairs = tokens * top
         tile_rows = getattr(library.load("moe", self.suffix), f"nva_moe_tile_rows_{self.suffix}")
-        bm = int(tile_rows(c_i64(pairs), c_i32(num_experts), c_i32(k), c_i32(ff)))
+        bm = int(tile_rows(_p(x), c_i64(xs), _p(up), _p(down), c_i64(tokens), c_i32(top), c_i32(num_experts), c_i32(k), c_i32(ff),
+                           c_i32(1 if gated else 0)))
         max_tiles = pairs // bm + num_experts
         ints = torch.empty(2 * pairs + 3 * max_tiles + 1, dtype=torch.int32, device=x.device)
         hidden = torch.empty((pairs, ff), dtype=x.dtype, device=x.device)
