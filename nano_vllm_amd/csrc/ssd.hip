@@ -98,19 +98,20 @@ ssd_conv_kernel(const T* __restrict__ proj, int64_t stride, int col0, int channe
     }
 }
 
-// The kept inputs of the requests that bring more than one token: the last K - 1 inputs of the portion,
+// The kept inputs of the requests that bring `fewest` tokens or more: the last K - 1 inputs of the portion,
 // or, where the portion is shorter, the old ones moved on.  A thread per (request, channel) reads all it
 // needs before it writes.
 template <typename T>
 __global__ void __launch_bounds__(256)
 ssd_conv_state_kernel(const T* __restrict__ proj, int64_t stride, int col0, int channels, int taps,
                       float* __restrict__ conv_state, const int32_t* __restrict__ cu_seqlens,
-                      const int32_t* __restrict__ seq_starts, const int32_t* __restrict__ state_slots, int first_seq) {
+                      const int32_t* __restrict__ seq_starts, const int32_t* __restrict__ state_slots, int first_seq,
+                      int fewest) {
     const int s = first_seq + blockIdx.y;
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= channels) return;
     const int begin = cu_seqlens[s], n = cu_seqlens[s + 1] - begin;
-    if (n <= 1) return;
+    if (n < fewest) return;
     const bool carried = seq_starts[s] > 0;
     const int hist = taps - 1;
     float* kept = conv_state + ((int64_t)state_slots[s] * channels + c) * hist;
@@ -621,6 +622,479 @@ ssd_finish_kernel(const float* __restrict__ y, const T* __restrict__ proj, int64
     }
 }
 
+#if defined(NVA_BF16)
+// ---------------------------------------------------------------------------- portions of bfloat16 models, as products
+// A portion's tokens in sub-blocks of 64.  With cum_t the sum of the log-decays of a sub-block's tokens up to t, E the
+// state before it and S the state after it,
+//     y_t = exp(cum_t) E^T C_t + sum over s <= t of [exp(cum_t - cum_s) dt_s (C_t . B_s) + (s == t) D] x_s
+//     S   = exp(cum_last) E + sum over s of exp(cum_last - cum_s) dt_s B_s x_s^T
+// and every sum is a product on the matrix cores.  B, C and x are bfloat16 (the convolution's output, rounded once); what
+// meets them (the weighted scores, the weighted x, the state) is float and enters as the sum of three bfloat16 parts, which
+// hold all its 24 bits: products of bfloat16 numbers are exact in the float accumulators, so the sums are those of float
+// operands, at 3/16 of a float product's time.  Every exponent is a difference of sums of logarithms that is <= 0.
+//
+// The convolution leaves B and C as rows [token][channel] and x and B in pieces of 8 tokens of one channel
+// [piece][channel][8 tokens], which are the operands of the products whose sum runs over tokens, straight from global
+// memory.  A portion's pieces are counted from its own first token: piece 0 of request s is cu_seqlens[s] / 8 + s.
+//
+// A unit is a run of up to block_tokens tokens of one portion (units[u] = request counted from num_single, first token,
+// tokens, units of the portion); a workgroup takes a unit, a head and 64 columns, its state in registers.  A portion of one
+// unit goes from its request's state to its new state in one pass (ssd_out).  The units of longer ones run side by side:
+// ssd_ends makes every unit's end state from a zero state (the first from the request's), ssd_link the true states, and
+// ssd_out the outputs.
+//
+// 64 heads of 64 columns, a state of 128 rows, 2048 tokens, in units of 128: convolution 31 us, ends 32, link 15, outputs
+// 60, gate and norm 14, kept inputs 4: 156 us, where the recurrence on the vector units took 411 (convolution 73, blocks
+// 202, their chain 29, second pass 81, gate and norm 26) and blocks as float products 417.  The floor is about 150 MB of
+// projections, pieces, states and outputs, 29 us at 5.2 TB/s; the outputs' kernel is bound by its vector work (splits,
+// exponentials) beside 70 matrix instructions a wave and sub-block, two workgroups a CU by their LDS.
+typedef __attribute__((ext_vector_type(8))) __bf16 ssd_bf16x8;
+typedef __attribute__((ext_vector_type(4))) __bf16 ssd_bf16x4;
+typedef __attribute__((ext_vector_type(2))) __bf16 ssd_bf16x2;
+#define SSD_STRETCH 32        // tokens a thread of the convolution takes
+#define SSD_PIECE_TAPS 8      // taps it is built for
+
+__device__ __forceinline__ int64_t ssd_piece0(const int32_t* cu_seqlens, int s) { return cu_seqlens[s] / 8 + s; }
+
+// Two channels and 32 tokens a thread: every input asked for once.  The last block of columns makes the step sizes and
+// decays of every head instead.
+__global__ void __launch_bounds__(256)
+ssd_conv_pieces_kernel(const __bf16* __restrict__ proj, int64_t stride, int col0, int channels, int inner, int gn, int taps,
+                       const __bf16* __restrict__ conv_w, const __bf16* __restrict__ conv_b,
+                       const float* __restrict__ conv_state, const int32_t* __restrict__ cu_seqlens,
+                       const int32_t* __restrict__ seq_starts, const int32_t* __restrict__ state_slots, int first_seq,
+                       const int32_t* __restrict__ units, __bf16* __restrict__ rows, __bf16* __restrict__ pieces,
+                       float* __restrict__ dtd, int heads, int dt_col, const float* __restrict__ dt_bias,
+                       const float* __restrict__ a_log) {
+    const int u = blockIdx.z, s = first_seq + units[4 * u];
+    const int i0 = units[4 * u + 1] + blockIdx.y * SSD_STRETCH;            // the first token within the portion
+    const int end = units[4 * u + 1] + units[4 * u + 2];
+    if (i0 >= end) return;
+    const int count = min(SSD_STRETCH, end - i0);
+    const int64_t t0 = cu_seqlens[s];
+    if (blockIdx.x == gridDim.x - 1) {
+        for (int idx = threadIdx.x; idx < count * heads; idx += 256) {
+            const int64_t t = t0 + i0 + idx / heads;
+            const int h = idx % heads;
+            const float dt = ssd_softplus(to_float(proj[t * stride + dt_col + h]) + dt_bias[h]);
+            dtd[(t * heads + h) * 2] = dt;
+            dtd[(t * heads + h) * 2 + 1] = -expf(a_log[h]) * dt;
+        }
+        return;
+    }
+    const int c = (blockIdx.x * 256 + threadIdx.x) * 2;
+    if (c >= channels) return;
+    const int hist = taps - 1;
+    const bool carried = seq_starts[s] > 0;
+    constexpr int H = SSD_PIECE_TAPS - 1;
+    float in0[H + SSD_STRETCH], in1[H + SSD_STRETCH];                      // token i0 - H + j of channels c and c + 1
+    const __bf16* src = proj + (t0 + i0) * stride + col0 + c;
+    ssd_bf16x2 v[H + SSD_STRETCH];
+#pragma unroll
+    for (int j = 0; j < H + SSD_STRETCH; ++j) {
+        const int i = min(max(i0 + j - H, 0), end - 1) - i0;               // (kept inside the portion)
+        v[j] = *reinterpret_cast<const ssd_bf16x2*>(src + (int64_t)i * stride);
+    }
+#pragma unroll
+    for (int j = 0; j < H + SSD_STRETCH; ++j) {
+        in0[j] = to_float(v[j][0]);
+        in1[j] = to_float(v[j][1]);
+    }
+    if (i0 < H) {                                                          // before the portion: what the request kept, or zeros
+        const float* kept = conv_state + ((int64_t)state_slots[s] * channels + c) * hist;
+#pragma unroll
+        for (int j = 0; j < H; ++j) {
+            const int i = i0 + j - H;
+            if (i < 0) {
+                const bool have = carried && hist + i >= 0;
+                in0[j] = have ? kept[hist + i] : 0.f;
+                in1[j] = have ? kept[hist + hist + i] : 0.f;
+            }
+        }
+    }
+    float w0[SSD_PIECE_TAPS], w1[SSD_PIECE_TAPS];                          // tap j reads the input H - j tokens back; the earliest are zero
+#pragma unroll
+    for (int j = 0; j < SSD_PIECE_TAPS; ++j) {
+        const int tap = j - (SSD_PIECE_TAPS - taps);
+        w0[j] = tap >= 0 ? to_float(conv_w[(int64_t)c * taps + tap]) : 0.f;
+        w1[j] = tap >= 0 ? to_float(conv_w[(int64_t)(c + 1) * taps + tap]) : 0.f;
+    }
+    const float b0 = to_float(conv_b[c]), b1 = to_float(conv_b[c + 1]);
+    const int piece_channels = inner + gn;
+    __bf16* pc = pieces + ((ssd_piece0(cu_seqlens, s) + i0 / 8) * piece_channels + c) * 8;
+    const bool as_row = c >= inner, as_piece = c < piece_channels;
+#pragma unroll
+    for (int q = 0; q < SSD_STRETCH / 8; ++q) {
+        if (8 * q >= count) break;
+        ssd_bf16x8 p0, p1;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int i = 8 * q + e;
+            float s0 = b0, s1 = b1;
+#pragma unroll
+            for (int j = 0; j < SSD_PIECE_TAPS; ++j)
+                if (j >= SSD_PIECE_TAPS - taps) {                          // (a tap that is not there adds nothing, not 0 times an infinity)
+                    s0 += w0[j] * in0[i + j];
+                    s1 += w1[j] * in1[i + j];
+                }
+            const bool there = i < count;
+            p0[e] = (__bf16)(there ? ssd_silu(s0) : 0.f);
+            p1[e] = (__bf16)(there ? ssd_silu(s1) : 0.f);
+            if (as_row && there) {
+                ssd_bf16x2 r = {p0[e], p1[e]};
+                *reinterpret_cast<ssd_bf16x2*>(rows + (t0 + i0 + i) * channels + c) = r;
+            }
+        }
+        if (as_piece) {
+            *reinterpret_cast<ssd_bf16x8*>(pc + (int64_t)q * piece_channels * 8) = p0;
+            *reinterpret_cast<ssd_bf16x8*>(pc + (int64_t)q * piece_channels * 8 + 8) = p1;
+        }
+    }
+}
+
+struct SsdUnitArgs {
+    const __bf16* rows; const __bf16* pieces; int channels, inner, gn;
+    const float* dtd; int heads, vdim, groups;
+    const float* d_skip; float* state;
+    const int32_t *cu_seqlens, *seq_starts, *state_slots; int first_seq;
+    const int32_t* units; float* block_states; float* totals; float* y;
+};
+
+// v as the sum of three bfloat16 numbers, eight values of v a call.
+__device__ __forceinline__ void ssd_split(const float (&v)[8], ssd_bf16x8 (&part)[3]) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        float r = v[j];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            part[q][j] = (__bf16)r;
+            r -= (float)part[q][j];
+        }
+        // (an infinity or NaN stays what it is; its remainder is no number and must not be added to it)
+        if (!(fabsf((float)part[0][j]) < INFINITY)) part[1][j] = part[2][j] = (__bf16)0.f;
+    }
+}
+
+// A sub-block's log-decays summed up to each token and its step sizes, one token a lane (zero beyond n).
+__device__ __forceinline__ void ssd_steps(const SsdUnitArgs& a, int64_t t0, int n, int h, int lane, float& dt, float& cum) {
+    dt = cum = 0.f;
+    if (lane < n) {
+        const float2 v = *reinterpret_cast<const float2*>(a.dtd + ((t0 + lane) * a.heads + h) * 2);
+        dt = v.x;
+        cum = v.y;
+    }
+#pragma unroll
+    for (int off = 1; off < NVA_WAVE; off <<= 1) {
+        const float up = __shfl_up(cum, off, NVA_WAVE);
+        if (lane >= off) cum += up;
+    }
+}
+
+// S <- exp(cum_last) S + sum of w_s B_s x_s^T over a sub-block of n tokens, w in LDS; a wave's tiles: columns 32 pi ...,
+// state rows 32 (first + 2 q) ...
+template <int NT>
+__device__ __forceinline__ void ssd_advance(const SsdUnitArgs& a, const __bf16* pieces, int n, int x_col, int b_col, int first,
+                                            const float* w_s, float keep, int lane, ssd_f32x16 (&S)[(NT + 1) / 2]) {
+    const int i = lane % 32, half = lane / 32;
+    const int64_t piece_stride = (int64_t)(a.inner + a.gn) * 8;
+#pragma unroll
+    for (int q = 0; q < (NT + 1) / 2; ++q)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) S[q][v] *= keep;
+    const ssd_bf16x8 zero = {};
+    ssd_bf16x8 xp[4], bp[4][(NT + 1) / 2];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+        const int piece = 2 * ks + half;
+        const bool there = 8 * piece < n;
+        const __bf16* p = pieces + (there ? piece : 0) * piece_stride;
+        xp[ks] = there ? *reinterpret_cast<const ssd_bf16x8*>(p + (int64_t)(x_col + i) * 8) : zero;
+#pragma unroll
+        for (int q = 0; q < (NT + 1) / 2; ++q)
+            bp[ks][q] = there && first + 2 * q < NT ? *reinterpret_cast<const ssd_bf16x8*>(p + (int64_t)(b_col + 32 * (first + 2 * q) + i) * 8) : zero;
+    }
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+        float w[8], wx[8];
+        load8(w_s + 16 * ks + 8 * half, w);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) wx[j] = w[j] * (float)xp[ks][j];
+        ssd_bf16x8 part[3];
+        ssd_split(wx, part);
+#pragma unroll
+        for (int q = 0; q < (NT + 1) / 2; ++q) {
+            if (first + 2 * q >= NT) continue;
+#pragma unroll
+            for (int r = 2; r >= 0; --r) S[q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bp[ks][q], part[r], S[q], 0, 0, 0);
+        }
+    }
+}
+
+template <int NT>
+__device__ __forceinline__ void ssd_move_state(float* at, int vdim, int col, int first, int lane, ssd_f32x16 (&S)[(NT + 1) / 2], bool store) {
+    const int i = lane % 32, half = lane / 32;
+#pragma unroll
+    for (int q = 0; q < (NT + 1) / 2; ++q) {
+        if (first + 2 * q >= NT) continue;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            float* p = at + (int64_t)(32 * (first + 2 * q) + 8 * (v / 4) + 4 * half + v % 4) * vdim + col + i;
+            if (store) *p = S[q][v]; else S[q][v] = *p;
+        }
+    }
+}
+
+template <int NT>
+__global__ void __launch_bounds__(256)
+ssd_ends_kernel(const SsdUnitArgs a) {
+    __shared__ __attribute__((aligned(16))) float w_s[4][64];
+    const int u = blockIdx.z, h = blockIdx.y, n_state = 32 * NT;
+    if (a.units[4 * u + 3] <= 1) return;
+    const int s = a.first_seq + a.units[4 * u], start = a.units[4 * u + 1], tokens = a.units[4 * u + 2];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / NVA_WAVE), lane = threadIdx.x % NVA_WAVE;
+    const int first = wave / 2, col = blockIdx.x * 64 + 32 * (wave % 2), g = h / (a.heads / a.groups);
+    const int64_t t0 = a.cu_seqlens[s] + start;
+    const __bf16* pieces = a.pieces + (ssd_piece0(a.cu_seqlens, s) + start / 8) * (a.inner + a.gn) * 8;
+    ssd_f32x16 S[(NT + 1) / 2];
+#pragma unroll
+    for (int q = 0; q < (NT + 1) / 2; ++q)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) S[q][v] = 0.f;
+    if (start == 0 && a.seq_starts[s] > 0)
+        ssd_move_state<NT>(a.state + ((int64_t)a.state_slots[s] * a.heads + h) * n_state * a.vdim, a.vdim, col, first, lane, S, false);
+    float total = 0.f;
+    for (int i0 = 0; i0 < tokens; i0 += 64) {
+        const int n = min(64, tokens - i0);
+        float dt, cum;
+        ssd_steps(a, t0 + i0, n, h, lane, dt, cum);
+        const float last = __shfl(cum, 63, NVA_WAVE);
+        w_s[wave][lane] = expf(last - cum) * dt;
+        total += last;
+        ssd_advance<NT>(a, pieces + (int64_t)(i0 / 8) * (a.inner + a.gn) * 8, n, h * a.vdim + col, a.inner + g * n_state, first,
+                        w_s[wave], expf(last), lane, S);
+    }
+    ssd_move_state<NT>(a.block_states + ((int64_t)u * a.heads + h) * n_state * a.vdim, a.vdim, col, first, lane, S, true);
+    if (threadIdx.x == 0 && blockIdx.x == 0) a.totals[u * a.heads + h] = total;
+}
+
+// The true states: block_states[u] <- exp(total of u) block_states[u - 1] + block_states[u] along a portion; the request
+// takes the last, whose place takes the state the request had, for the portion's first unit to start from.
+__global__ void __launch_bounds__(256)
+ssd_link_kernel(float* __restrict__ block_states, const float* __restrict__ totals, float* __restrict__ state,
+                const int32_t* __restrict__ chains, const int32_t* __restrict__ state_slots, int first_seq, int heads, int per_head) {
+    const int c = blockIdx.z, h = blockIdx.y;
+    const int e = (blockIdx.x * blockDim.x + threadIdx.x) * 4;
+    if (e >= per_head) return;
+    const int u0 = chains[4 * c], blocks = chains[4 * c + 1], s = first_seq + chains[4 * c + 2];
+    const int64_t step = (int64_t)heads * per_head;
+    float* at = block_states + (int64_t)u0 * step + (int64_t)h * per_head + e;
+    float* own = state + ((int64_t)state_slots[s] * heads + h) * per_head + e;
+    const float4 before = *reinterpret_cast<const float4*>(own);
+    float4 carry = *reinterpret_cast<const float4*>(at);
+    constexpr int AHEAD = 8;                               // units asked for before any is used
+    for (int b0 = 1; b0 < blocks; b0 += AHEAD) {
+        float4 v[AHEAD];
+        float k[AHEAD];
+#pragma unroll
+        for (int q = 0; q < AHEAD; ++q) {
+            const int b = min(b0 + q, blocks - 1);
+            v[q] = *reinterpret_cast<const float4*>(at + b * step);
+            k[q] = expf(totals[(u0 + b) * heads + h]);
+        }
+#pragma unroll
+        for (int q = 0; q < AHEAD; ++q) {
+            if (b0 + q >= blocks) break;
+            carry = make_float4(k[q] * carry.x + v[q].x, k[q] * carry.y + v[q].y, k[q] * carry.z + v[q].z, k[q] * carry.w + v[q].w);
+            if (b0 + q < blocks - 1) *reinterpret_cast<float4*>(at + (b0 + q) * step) = carry;
+        }
+    }
+    *reinterpret_cast<float4*>(own) = carry;
+    *reinterpret_cast<float4*>(at + (blocks - 1) * step) = before;
+}
+
+// LDS: the state in three parts [64 columns][32 NT rows] and the weighted scores in three parts [64 t][64 s], 16-byte pieces
+// of a row turned by the row's number so that the rows of a read lie in different banks; a sub-block's steps.
+template <int NT> __device__ __forceinline__ uint32_t ssd_e_at(int p, int piece) {
+    constexpr int PIECES = 4 * NT;
+    const int turn = PIECES >= 16 ? p % 16 : PIECES == 8 ? p / 2 % 8 : p / 4 % 4;
+    return (uint32_t)(p * PIECES + (piece ^ turn)) * 16;
+}
+__device__ __forceinline__ uint32_t ssd_m_at(int t, int piece) { return (uint32_t)(t * 8 + (piece ^ (t / 2 % 8))) * 16; }
+
+template <int NT>
+__global__ void __launch_bounds__(256, 2)
+ssd_out_kernel(const SsdUnitArgs a) {
+    constexpr int E_BYTES = 64 * 32 * NT * 2, M_BYTES = 64 * 64 * 2;
+    extern __shared__ __attribute__((aligned(16))) char ssd_lds[];
+    char* e_s = ssd_lds;                                   // three parts
+    char* m_s = ssd_lds + 3 * E_BYTES;                     // three parts
+    float* w_s = (float*)(m_s + 3 * M_BYTES);              // [4 waves][64]
+    float* cum_s = w_s + 4 * 64;                           // [4 waves][64]
+    const int u = blockIdx.z, h = blockIdx.y, n_state = 32 * NT;
+    const int s = a.first_seq + a.units[4 * u], start = a.units[4 * u + 1], tokens = a.units[4 * u + 2], count = a.units[4 * u + 3];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / NVA_WAVE), lane = threadIdx.x % NVA_WAVE;
+    const int i = lane % 32, half = lane / 32;
+    const int first = wave / 2, pi = wave % 2, ti = wave / 2, col = blockIdx.x * 64 + 32 * pi, g = h / (a.heads / a.groups);
+    const int64_t t0 = a.cu_seqlens[s] + start;
+    const int64_t piece_stride = (int64_t)(a.inner + a.gn) * 8;
+    const __bf16* pieces = a.pieces + (ssd_piece0(a.cu_seqlens, s) + start / 8) * piece_stride;
+    const int64_t per_head = (int64_t)n_state * a.vdim;
+    float* own = a.state + ((int64_t)a.state_slots[s] * a.heads + h) * per_head;
+    ssd_f32x16 S[(NT + 1) / 2];
+#pragma unroll
+    for (int q = 0; q < (NT + 1) / 2; ++q)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) S[q][v] = 0.f;
+    const bool has_start = start > 0 || a.seq_starts[s] > 0;
+    if (has_start) {
+        // the unit before's end; for a portion's first unit the request's state, which the link left in the last unit's place
+        float* from = count == 1 ? own : a.block_states + ((int64_t)(start > 0 ? u - 1 : u + count - 1) * a.heads + h) * per_head;
+        ssd_move_state<NT>(from, a.vdim, col, first, lane, S, false);
+    }
+    const float skip = a.d_skip[h];
+    for (int i0 = 0; i0 < tokens; i0 += 64) {
+        const int n = min(64, tokens - i0);
+        const __bf16* px = pieces + (int64_t)(i0 / 8) * piece_stride;
+        // C of this wave's 32 tokens and B of the tokens it meets first; rows beyond the portion are its last one again
+        const __bf16* c_row = a.rows + (t0 + i0 + min(32 * ti + i, n - 1)) * a.channels + a.inner + a.gn + g * n_state + 8 * half;
+        const int si = ti == 0 ? 0 : 1 - pi;               // the tile of scores this wave makes (wave 1 makes none)
+        const __bf16* b_row = a.rows + (t0 + i0 + min(32 * si + i, n - 1)) * a.channels + a.inner + g * n_state + 8 * half;
+        ssd_bf16x8 cf[2 * NT];
+#pragma unroll
+        for (int ks = 0; ks < 2 * NT; ++ks) cf[ks] = *reinterpret_cast<const ssd_bf16x8*>(c_row + 16 * ks);
+        float dt, cum;
+        ssd_steps(a, t0 + i0, n, h, lane, dt, cum);
+        const float last = __shfl(cum, 63, NVA_WAVE);
+        float* w = w_s + 64 * wave;
+        float* cw = cum_s + 64 * wave;
+        w[lane] = dt;
+        cw[lane] = cum;
+        // ---- the state before the sub-block, in parts: this wave's tiles hold rows 8 (v / 4) + 4 half + v % 4 of column i
+#pragma unroll
+        for (int q = 0; q < (NT + 1) / 2; ++q) {
+            if (first + 2 * q >= NT) continue;
+#pragma unroll
+            for (int v8 = 0; v8 < 2; ++v8) {
+                float val[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) val[j] = S[q][8 * v8 + j];
+                ssd_bf16x8 part[3];
+                ssd_split(val, part);
+#pragma unroll
+                for (int r = 0; r < 3; ++r)
+#pragma unroll
+                    for (int v4 = 0; v4 < 2; ++v4) {
+                        ssd_bf16x4 four = {part[r][4 * v4], part[r][4 * v4 + 1], part[r][4 * v4 + 2], part[r][4 * v4 + 3]};
+                        *reinterpret_cast<ssd_bf16x4*>(e_s + r * E_BYTES + ssd_e_at<NT>(32 * pi + i, 4 * (first + 2 * q) + 2 * v8 + v4) + 8 * half) = four;
+                    }
+            }
+        }
+        // ---- the scores, transposed: rows s, columns t, so that a lane holds four neighbouring s of one t
+        if (wave != 1) {
+            ssd_f32x16 acc;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[v] = 0.f;
+            // (C as the other operand: this wave's own tile of tokens)
+#pragma unroll
+            for (int ks = 0; ks < 2 * NT; ++ks)
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const ssd_bf16x8*>(b_row + 16 * ks), cf[ks], acc, 0, 0, 0);
+            const int t = 32 * ti + i;
+            const float cum_t = cw[t];
+#pragma unroll
+            for (int v8 = 0; v8 < 2; ++v8) {
+                float val[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const int v = 8 * v8 + j, sc = 32 * si + 8 * (v / 4) + 4 * half + v % 4;
+                    val[j] = sc <= t ? acc[v] * expf(cum_t - cw[sc]) * w[sc] + (sc == t ? skip : 0.f) : 0.f;
+                }
+                ssd_bf16x8 part[3];
+                ssd_split(val, part);
+#pragma unroll
+                for (int r = 0; r < 3; ++r)
+#pragma unroll
+                    for (int v4 = 0; v4 < 2; ++v4) {
+                        ssd_bf16x4 four = {part[r][4 * v4], part[r][4 * v4 + 1], part[r][4 * v4 + 2], part[r][4 * v4 + 3]};
+                        *reinterpret_cast<ssd_bf16x4*>(m_s + r * M_BYTES + ssd_m_at(t, 4 * si + 2 * v8 + v4) + 8 * half) = four;
+                    }
+            }
+        }
+        __syncthreads();
+        // ---- y: what the state before adds, times each token's decay up to it, then the sub-block's own tokens
+        ssd_f32x16 y;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) y[v] = 0.f;
+        if (has_start || i0 > 0) {
+#pragma unroll
+            for (int ks = 0; ks < 2 * NT; ++ks)
+#pragma unroll
+                for (int r = 2; r >= 0; --r) {
+                    const ssd_bf16x8 ef = *reinterpret_cast<const ssd_bf16x8*>(e_s + r * E_BYTES + ssd_e_at<NT>(32 * pi + i, 2 * ks + half));
+                    y = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cf[ks], ef, y, 0, 0, 0);
+                }
+#pragma unroll
+            for (int v = 0; v < 16; ++v) y[v] *= expf(cw[32 * ti + 8 * (v / 4) + 4 * half + v % 4]);
+        }
+        const ssd_bf16x8 zero = {};
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+            if (ks >= 2 * (ti + 1)) break;
+            const int piece = 2 * ks + half;
+            const ssd_bf16x8 xf = 8 * piece < n ? *reinterpret_cast<const ssd_bf16x8*>(px + piece * piece_stride + (int64_t)(h * a.vdim + col + i) * 8) : zero;
+#pragma unroll
+            for (int r = 2; r >= 0; --r) {
+                const ssd_bf16x8 mf = *reinterpret_cast<const ssd_bf16x8*>(m_s + r * M_BYTES + ssd_m_at(32 * ti + i, piece));
+                y = __builtin_amdgcn_mfma_f32_32x32x16_bf16(mf, xf, y, 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            const int t = 32 * ti + 8 * (v / 4) + 4 * half + v % 4;
+            if (t < n) a.y[(t0 + i0 + t) * a.inner + h * a.vdim + col + i] = y[v];
+        }
+        // ---- the state after the sub-block, where somebody reads it
+        if (i0 + 64 < tokens || count == 1) {
+            w[lane] = expf(last - cum) * dt;
+            ssd_advance<NT>(a, px, n, h * a.vdim + col, a.inner + g * n_state, first, w, expf(last), lane, S);
+        }
+        __syncthreads();
+    }
+    if (count == 1) ssd_move_state<NT>(own, a.vdim, col, first, lane, S, true);
+}
+
+// Gate and norm of rows whose parts are 256 threads times 8, or 16, numbers: read once, kept in registers.
+template <int PER>
+__global__ void __launch_bounds__(256)
+ssd_finish8_kernel(const float* __restrict__ y, const __bf16* __restrict__ proj, int64_t stride, const float* __restrict__ weight,
+                   int inner, float eps, __bf16* __restrict__ out, int64_t out_stride) {
+    __shared__ float scratch[16];
+    const int64_t t = blockIdx.x;
+    const int at = blockIdx.y * 256 * 8 * PER + threadIdx.x * 8;
+    float v[PER][8], ss = 0.f;
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+        float z[8];
+        load8(y + t * inner + at + q * 2048, v[q]);
+        load8(proj + t * stride + at + q * 2048, z);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            v[q][j] *= ssd_silu(z[j]);
+            ss += v[q][j] * v[q][j];
+        }
+    }
+    ss = block_sum(ss, scratch);
+    const float scale = rsqrtf(ss / (float)(256 * 8 * PER) + eps);
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+        float w[8];
+        load8(weight + at + q * 2048, w);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[q][j] = v[q][j] * scale * w[j];
+        store8(out + t * out_stride + at + q * 2048, v[q]);
+    }
+}
+#endif
+
 struct ScanArgs {
     const elem_t* conv; int channels; const float* bc; int np; const float* dtd; int heads, vdim, n_state, groups;
     const float *a_log, *d_skip; float* state; const int32_t *cu, *starts, *slots;
@@ -631,6 +1105,16 @@ struct ScanArgs {
 // share a column) hold, the state's rounded up.
 static int ssd_padded_rows(int n_state) {
     return n_state <= 16 ? 16 : n_state <= 32 ? 32 : n_state <= 64 ? 64 : n_state <= 128 ? 128 : 256;
+}
+// Whether portions of these sizes run as products on the matrix cores (the caller then brings `pieces`, elements
+// [tokens / 8 + requests + 1][H P + G N][8], `totals`, float [units][H], and units of whole 64 tokens for every portion).
+NVA_EXPORT int NVA_NAME(nva_state_space_products)(const void* proj, int64_t stride, int heads, int vdim, int n_state, int groups, int taps) {
+#if defined(NVA_BF16)
+    return vdim % 64 == 0 && (n_state == 32 || n_state == 64 || n_state == 128) && taps <= SSD_PIECE_TAPS && stride % 2 == 0 &&
+           nva_aligned(proj, 4) && heads % groups == 0;
+#else
+    return 0;
+#endif
 }
 NVA_EXPORT int NVA_NAME(nva_state_space_padded_rows)(int n_state) { return ssd_padded_rows(n_state); }
 
@@ -664,7 +1148,7 @@ NVA_EXPORT int NVA_NAME(nva_state_space)(const void* proj, int64_t stride, void*
                                          const void* conv_b, const float* dt_bias, const float* a_log, const float* d_skip,
                                          const float* norm_w, int norm_groups, float eps, const int32_t* units,
                                          int64_t n_units, const int32_t* chains, int64_t n_chains, int block_tokens,
-                                         float* block_states, int shape, hipStream_t stream) {
+                                         float* block_states, int shape, void* pieces, float* totals, hipStream_t stream) {
     if (tokens == 0) return 0;
     if (tokens < 0 || seqs <= 0 || seqs > 65535 || num_single < 0 || num_single > seqs || slots <= 0)
         return nva_fail("state_space: bad counts tokens=%lld requests=%lld", (long long)tokens, (long long)seqs);
@@ -679,20 +1163,34 @@ NVA_EXPORT int NVA_NAME(nva_state_space)(const void* proj, int64_t stride, void*
     if (!proj || !conv_out || !bc || !dtd || !y_raw || !out || !state || (!conv_state && taps > 1) || !token_seq || !cu_seqlens || !seq_starts ||
         !state_slots || !conv_w || !conv_b || !dt_bias || !a_log || !d_skip || !norm_w)
         return nva_fail("state_space: a tensor is missing");
-    if (n_chains && (!units || !chains || !block_states || !cum || block_tokens <= 0 || n_units * ((block_tokens + 63) / 64) > 65535))
+    if (n_chains && (!units || !chains || !block_states || (!cum && !pieces) || block_tokens <= 0 || n_units * ((block_tokens + 63) / 64) > 65535))
         return nva_fail("state_space: blocks need their scratch and their size");
     const elem_t* pj = (const elem_t*)proj;
     if (tokens > 0x7fffffff || (channels + 255) / 256 > 65535) return nva_fail("state_space: too many tokens or channels");
+    const bool as_products = pieces != nullptr;                            // portions: nva_state_space_products said yes
+    if (as_products && (!units || n_units <= 0 || n_units > 65535 || !NVA_NAME(nva_state_space_products)(proj, stride, heads, vdim, n_state, groups, taps) ||
+                        (n_chains && (!totals || !block_states)) || block_tokens % 64))
+        return nva_fail("state_space: portions as products need their units and scratch");
+    const int64_t conv_tokens = as_products ? num_single : tokens;         // (single tokens come first)
     const int per_thread = tokens >= 1024 ? SSD_CONV_TOKENS : 1;
+    if (conv_tokens > 0)
     hipLaunchKernelGGL((ssd_conv_kernel<elem_t>),
-                       dim3((unsigned)((tokens + per_thread - 1) / per_thread), (channels + 255) / 256), dim3(256), 0, stream, pj,
+                       dim3((unsigned)((conv_tokens + per_thread - 1) / per_thread), (channels + 255) / 256), dim3(256), 0, stream, pj,
                        stride, inner, channels, taps, (const elem_t*)conv_w, (const elem_t*)conv_b, conv_state, token_seq,
                        cu_seqlens, seq_starts, state_slots, (elem_t*)conv_out, bc, ssd_padded_rows(n_state), n_state, groups, dtd,
-                       heads, inner + channels, dt_bias, a_log, tokens, per_thread);
+                       heads, inner + channels, dt_bias, a_log, conv_tokens, per_thread);
+#if defined(NVA_BF16)
+    if (as_products)
+        hipLaunchKernelGGL(ssd_conv_pieces_kernel,
+                           dim3((unsigned)((channels + 511) / 512 + 1), (unsigned)(block_tokens / SSD_STRETCH), (unsigned)n_units), dim3(256), 0,
+                           stream, pj, stride, inner, channels, inner, groups * n_state, taps, (const __bf16*)conv_w, (const __bf16*)conv_b,
+                           conv_state, cu_seqlens, seq_starts, state_slots, (int)num_single, units, (__bf16*)conv_out, (__bf16*)pieces,
+                           dtd, heads, inner + channels, dt_bias, a_log);
+#endif
     if (seqs > num_single && taps > 1)
         hipLaunchKernelGGL((ssd_conv_state_kernel<elem_t>), dim3((channels + 255) / 256, (unsigned)(seqs - num_single)),
                            dim3(256), 0, stream, pj, stride, inner, channels, taps, conv_state, cu_seqlens, seq_starts,
-                           state_slots, (int)num_single);
+                           state_slots, (int)num_single, as_products ? 1 : 2);
     const ScanArgs args{(const elem_t*)conv_out, channels, bc, ssd_padded_rows(n_state), dtd, heads, vdim, n_state, groups,
                         a_log, d_skip, state, cu_seqlens, seq_starts, state_slots, block_states, cum, y_raw};
     // a thread holds up to 64 rows of a column of S; a state of more rows is shared out over 2 or 4 lanes
@@ -714,6 +1212,31 @@ NVA_EXPORT int NVA_NAME(nva_state_space)(const void* proj, int64_t stride, void*
         else if (num_single)
             scan((unsigned)num_single, 0, nullptr, 0);
     };
+#if defined(NVA_BF16)
+    if (as_products) {
+        single();
+        const SsdUnitArgs ua{(const __bf16*)conv_out, (const __bf16*)pieces, channels, inner, groups * n_state, dtd, heads, vdim, groups,
+                             d_skip, state, cu_seqlens, seq_starts, state_slots, (int)num_single, units, block_states, totals, y_raw};
+        const dim3 grid((unsigned)(vdim / 64), (unsigned)heads, (unsigned)n_units);
+#define SSD_PRODUCTS(NT)                                                                                                      \
+        do {                                                                                                                  \
+            const int lds = 3 * (64 * 32 * NT * 2 + 64 * 64 * 2) + 2 * 4 * 64 * 4;                                            \
+            if (hipFuncSetAttribute((const void*)ssd_out_kernel<NT>, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) \
+                return nva_fail("state_space: %d bytes of LDS are not to be had", lds);                                       \
+            if (n_chains) {                                                                                                   \
+                hipLaunchKernelGGL((ssd_ends_kernel<NT>), grid, dim3(256), 0, stream, ua);                                    \
+                hipLaunchKernelGGL(ssd_link_kernel, dim3((unsigned)((n_state * vdim / 4 + 255) / 256), (unsigned)heads, (unsigned)n_chains), \
+                                   dim3(256), 0, stream, block_states, totals, state, chains, state_slots, (int)num_single, heads, \
+                                   n_state * vdim);                                                                           \
+            }                                                                                                                 \
+            hipLaunchKernelGGL((ssd_out_kernel<NT>), grid, dim3(256), lds, stream, ua);                                       \
+        } while (0)
+        if (n_state == 32) SSD_PRODUCTS(1);
+        else if (n_state == 64) SSD_PRODUCTS(2);
+        else SSD_PRODUCTS(4);
+#undef SSD_PRODUCTS
+    } else
+#endif
     if (n_chains) {
         if (n_units <= 0 || n_units > 65535) return nva_fail("state_space: bad block count %lld", (long long)n_units);
         single();
@@ -765,6 +1288,15 @@ NVA_EXPORT int NVA_NAME(nva_state_space)(const void* proj, int64_t stride, void*
         }
     }
     const int group_size = inner / norm_groups;
+#if defined(NVA_BF16)
+    if ((group_size == 2048 || group_size == 4096) && stride % 8 == 0 && out_stride % 8 == 0 && nva_aligned(proj, 16) && nva_aligned(out, 16) &&
+        nva_aligned(y_raw, 32) && nva_aligned(norm_w, 32)) {
+        const auto kernel = group_size == 2048 ? ssd_finish8_kernel<1> : ssd_finish8_kernel<2>;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)tokens, norm_groups), dim3(256), 0, stream, y_raw, pj, stride, norm_w, inner, eps,
+                           (__bf16*)out, out_stride);
+        return nva_check_launch("state_space");
+    }
+#endif
     // (few tokens: more threads a row, so that a row's loads are on their way at once)
     hipLaunchKernelGGL((ssd_finish_kernel<elem_t>), dim3((unsigned)tokens, norm_groups),
                        dim3(tokens <= 64 && group_size >= 2048 ? 1024 : 256), 0, stream, y_raw, pj,

@@ -216,6 +216,26 @@ def state_space_blocks(q_lens, first_seq: int):
     return bt, units, chains
 
 
+def state_space_units(q_lens, first_seq: int, heads: int, cus: int):
+    """The step's portions cut into units for the state-space layer's products: (tokens of a unit, units, chains) as
+    retention_blocks gives them.  Units of 128 tokens (they run side by side, so many fill the GPU), twice as many and so on
+    while heads and units give every compute unit more than 2.5 workgroups: a unit's end state passes through memory.
+    64 heads (a state of 128 x 64), the mixer's time with units of 128, 256 and 512 tokens, in us: 1024 tokens 141, 158,
+    206; 2048 tokens 250, 241, 278; 4096 tokens 449, 441, 431; 8192 tokens 850, 820, 807."""
+    size = 128
+    while 2 * heads * sum((n + size - 1) // size for n in q_lens[first_seq:]) > 5 * cus and size < max(q_lens[first_seq:]):
+        size *= 2
+    units, chains = [], []
+    for s in range(first_seq, len(q_lens)):
+        n = q_lens[s]
+        count = (n + size - 1) // size
+        if count > 1:
+            chains += [len(units) // 4, count, s - first_seq, n - (count - 1) * size]
+        for u in range(count):
+            units += [s - first_seq, u * size, min(size, n - u * size), count]
+    return size, units, chains
+
+
 def prefill_tile_order(q_lens, starts, first_seq: int) -> list:
     """Flat [(request, row tile), ...] of the requests from `first_seq` on, from the tile that
     sees the most keys to the one that sees the fewest: the prefill attention kernel hands its
@@ -2087,27 +2107,35 @@ class HipKernels:
             bc.zero_()
         dtd = torch.empty((tokens, heads, 2), dtype=torch.float32, device=proj.device)
         # long portions are cut into blocks that run side by side (the same cut for every layer of the step)
-        units = chains = block_states = cum = None
+        units = chains = block_states = cum = pieces = totals = None
         n_units = n_chains = block_tokens = 0
         first = batch.num_decode
         if self.state_space_blocks_side_by_side and first < seqs:
+            takes = getattr(library.load("ssd", self.suffix), f"nva_state_space_products_{self.suffix}")
+            products = self.state_space_shape == 0 and bool(takes(_p(proj), c_i64(stride), c_i32(heads), c_i32(vdim), c_i32(n_state),
+                                                                  c_i32(groups), c_i32(taps)))
+            cut = state_space_units if products else state_space_blocks if self.state_space_shape == 6 else retention_blocks
+            given = (heads, self.cus) if products else ()
             kept = getattr(batch, "step_cache", None)
             if kept is None:
                 kept = batch.step_cache = {}
-            plan = kept.get(("state_space_blocks", first, self.state_space_shape == 6))
+            plan = kept.get((cut.__name__, first, *given))
             if plan is None:
-                block_tokens, flat_units, flat_chains = (state_space_blocks if self.state_space_shape == 6 else retention_blocks)(
-                    batch.q_lens, first)
-                if flat_chains:
+                block_tokens, flat_units, flat_chains = cut(batch.q_lens, first, *given)
+                if flat_chains or products:
                     both = torch.tensor(flat_units + flat_chains, dtype=torch.int32).to(proj.device, non_blocking=True)
                     plan = (len(flat_units) // 4, len(flat_chains) // 4, both[: len(flat_units)], both[len(flat_units):],
                             block_tokens)
                 else:
                     plan = (0, 0, None, None, 0)
-                kept[("state_space_blocks", first, self.state_space_shape == 6)] = plan
+                kept[(cut.__name__, first, *given)] = plan
             n_units, n_chains, units, chains, block_tokens = plan
             if n_chains:
                 block_states = torch.empty((n_units, heads, n_state, vdim), dtype=torch.float32, device=proj.device)
+            if products:
+                pieces = torch.empty((tokens // 8 + seqs + 1, inner + gn, 8), dtype=proj.dtype, device=proj.device)
+                totals = torch.empty((n_units, heads), dtype=torch.float32, device=proj.device)
+            elif n_chains:
                 cum = torch.empty((tokens, heads), dtype=torch.float32, device=proj.device)
         library.call("ssd", _suffix(proj), "nva_state_space", _p(proj), c_i64(stride), _p(conv_out), _p(bc), _p(dtd), _p(y_raw),
                      _p(cum), _p(out),
@@ -2116,7 +2144,7 @@ class HipKernels:
                      c_i64(first), c_i32(heads), c_i32(vdim), c_i32(n_state), c_i32(groups), c_i32(taps), _p(conv_w),
                      _p(conv_b), _p(dt_bias), _p(a_log), _p(d_skip), _p(norm_w), c_i32(norm_groups), c_f32(eps), _p(units),
                      c_i64(n_units), _p(chains), c_i64(n_chains), c_i32(block_tokens), _p(block_states),
-                     c_i32(self.state_space_shape),
+                     c_i32(self.state_space_shape), _p(pieces), _p(totals),
                      self._stream())
         return out
 
