@@ -222,6 +222,152 @@ paged_attention_merge_kernel(const float* __restrict__ part, int shares, T* __re
     }
 }
 
+#define ATT_SINGLE_WAVES 8
+#define ATT_SINGLE_PAIRS 16384     // (token, head) pairs up to which a workgroup takes each
+#define ATT_SINGLE_MAX_D 128
+#define ATT_V_LD 68               // floats of a channel's 64 keys in LDS: rows start in different banks
+
+// The same attention for few tokens, one workgroup of eight waves per (token, head) instead of one wave, with the
+// per-token kernel's arithmetic, operation for operation (equal bits): eight blocks of 64 keys at a time, a wave the scores of
+// one block; the running maximum passes over the blocks' maxima in order, and every block's weights are taken with the
+// maximum up to it; then the blocks' values go through LDS, all waves bringing the next block (whole tiles of 32 keys of a
+// channel, 16 bytes a lane) while the first two waves add up this one, a channel a thread, its keys in ascending order.
+// One wave alone waits for every batch of loads in turn.  16 heads of 128 floats, 8 kv heads, us with one wave / here: 1 token
+// of 1500 keys 218 / 83; 7 tokens of 50 to 1500 208 / 80; 2 of 8000 1141 / 426; 16 of 500 77 / 31; 64 of 500 146 / 116; 256 of
+// 300 to 600 770 / 596; 512 of 100 to 300 685 / 579; 1000 of 20 to 200 759 / 759: from there on the pairs fill the GPU.
+// No window, no sigmoid weights, head sizes up to 128, whole tiles of 32 keys in a page.
+template <typename T>
+__global__ void __launch_bounds__(ATT_SINGLE_WAVES * NVA_WAVE)
+paged_attention_single_kernel(const T* __restrict__ q, int64_t q_stride, T* __restrict__ out, int64_t out_stride,
+                              const T* __restrict__ k_cache, const T* __restrict__ v_cache,
+                              const int32_t* __restrict__ block_tables, int table_stride,
+                              const int32_t* __restrict__ token_seq, const int32_t* __restrict__ positions,
+                              int num_q_heads, int num_kv_heads, int head_dim, int v_dim, int page_size, float scale,
+                              int chunk, float softcap, const float* __restrict__ sinks, const float* __restrict__ head_gate,
+                              int32_t* error_flag) {
+    extern __shared__ __attribute__((aligned(16))) float v_s[];               // [2][ATT_SINGLE_MAX_D][ATT_V_LD]
+    __shared__ __attribute__((aligned(16))) float q_s[ATT_SINGLE_MAX_D];
+    __shared__ __attribute__((aligned(16))) float p_s[ATT_SINGLE_WAVES][NVA_WAVE];
+    __shared__ float max_s[ATT_SINGLE_WAVES], sum_s[ATT_SINGLE_WAVES];
+    const int64_t t = blockIdx.x;
+    const int h = blockIdx.y, kvh = h / (num_q_heads / num_kv_heads);
+    const int tid = threadIdx.x, wave = tid / NVA_WAVE, lane = tid % NVA_WAVE;
+    const int pos = positions[t];
+    const int first = nva_first_key(pos, 0, chunk);
+    const int32_t* table = block_tables + (int64_t)token_seq[t] * table_stride;
+    for (int d = tid; d < head_dim; d += blockDim.x) q_s[d] = to_float(q[t * q_stride + (int64_t)h * head_dim + d]);
+    constexpr int V4 = ATT_SINGLE_MAX_D * NVA_WAVE / 4 / (ATT_SINGLE_WAVES * NVA_WAVE);     // pieces of four keys a thread brings of a block
+    float vr[V4][4];
+    // a block's values: piece n is channel n / 8 of the first 32 keys' tile, then of the second's; four keys of it
+    auto fetch_v = [&](int base) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < V4; ++i) {
+            const int n = tid + i * ATT_SINGLE_WAVES * NVA_WAVE, tile = n / (ATT_SINGLE_MAX_D * 8), c = n % (ATT_SINGLE_MAX_D * 8) / 8;
+            const int j0 = base + 32 * tile;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) vr[i][e] = 0.f;
+            if (c >= v_dim || j0 > pos) continue;
+            const int page = table[j0 / page_size];
+            if (page < 0) continue;
+            const T* p = v_cache + ((int64_t)page * num_kv_heads + kvh) * v_dim * (int64_t)page_size +
+                         nva_v_offset(j0 % page_size, c, v_dim, 32) + 4 * (n % 8);
+            typedef __attribute__((ext_vector_type(4))) T t4;
+            const t4 v = *reinterpret_cast<const t4*>(p);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) vr[i][e] = to_float(v[e]);
+        }
+    };
+    auto put_v = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < V4; ++i) {
+            const int n = tid + i * ATT_SINGLE_WAVES * NVA_WAVE, tile = n / (ATT_SINGLE_MAX_D * 8), c = n % (ATT_SINGLE_MAX_D * 8) / 8;
+            *reinterpret_cast<float4*>(&v_s[(buf * ATT_SINGLE_MAX_D + c) * ATT_V_LD + 32 * tile + 4 * (n % 8)]) =
+                make_float4(vr[i][0], vr[i][1], vr[i][2], vr[i][3]);
+        }
+    };
+    float acc = 0.f, m_run = sinks ? sinks[h] : -INFINITY, l_run = sinks ? 1.f : 0.f;
+    __syncthreads();
+    for (int batch = first / NVA_WAVE * NVA_WAVE; batch <= pos; batch += ATT_SINGLE_WAVES * NVA_WAVE) {
+        const int blocks = min(ATT_SINGLE_WAVES, (pos - batch) / NVA_WAVE + 1);
+        const int j = batch + NVA_WAVE * wave + lane;
+        float s = -INFINITY;
+        if (j <= pos && j >= first) {
+            const int page = table[j / page_size];
+            if (page < 0) {
+                if (error_flag) atomicOr(error_flag, 2);      // a visible key has no page
+            } else {
+                const T* krow = k_cache + (((int64_t)page * num_kv_heads + kvh) * page_size + j % page_size) * head_dim;
+                float dot = 0.f;
+                for (int d0 = 0; d0 < head_dim; d0 += 64) {   // eight loads of eight on their way at once; the sum stays one chain
+                    float kk[8][8];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u)
+                        if (d0 + 8 * u < head_dim) load8(krow + d0 + 8 * u, kk[u]);
+#pragma unroll
+                    for (int u = 0; u < 8; ++u)
+                        if (d0 + 8 * u < head_dim)
+#pragma unroll
+                            for (int e = 0; e < 8; ++e) dot += q_s[d0 + 8 * u + e] * kk[u][e];
+                }
+                s = dot * scale;
+                if (softcap > 0.f) s = softcap * tanhf(s / softcap);
+            }
+        }
+        fetch_v(batch);
+        const float top = wave_max(s);
+        if (lane == 0) max_s[wave] = top;
+        __syncthreads();
+        // the running maximum before and with this wave's block, and what each block's predecessors are rescaled by
+        float m = m_run, m_mine = m_run, corr[ATT_SINGLE_WAVES];
+#pragma unroll
+        for (int b = 0; b < ATT_SINGLE_WAVES; ++b) {
+            const float m_new = b < blocks ? fmaxf(m, max_s[b]) : m;
+            corr[b] = m == -INFINITY ? 0.f : nva_exp(m - m_new);
+            if (b == wave) m_mine = m_new;
+            m = m_new;
+        }
+        m_run = m;
+        const float p = s == -INFINITY ? 0.f : nva_exp(s - m_mine);
+        const float sum = wave_sum(p);
+        p_s[wave][lane] = p;
+        if (lane == 0) sum_s[wave] = sum;
+        put_v(0);
+        __syncthreads();
+#pragma unroll
+        for (int b = 0; b < ATT_SINGLE_WAVES; ++b) {
+            if (b >= blocks) break;
+            if (b + 1 < blocks) fetch_v(batch + NVA_WAVE * (b + 1));
+            l_run = l_run * corr[b] + sum_s[b];
+            if (tid < v_dim) {
+                acc *= corr[b];
+                const int base = batch + NVA_WAVE * b, valid = min(NVA_WAVE, pos - base + 1);
+                const float* vc = &v_s[((b & 1) * ATT_SINGLE_MAX_D + tid) * ATT_V_LD];
+                auto add_keys = [&](int k0) __attribute__((always_inline)) {
+                    float vv[16], pp[16];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        const float4 v = *reinterpret_cast<const float4*>(vc + k0 + 4 * u), w = *reinterpret_cast<const float4*>(&p_s[b][k0 + 4 * u]);
+                        vv[4 * u] = v.x, vv[4 * u + 1] = v.y, vv[4 * u + 2] = v.z, vv[4 * u + 3] = v.w;
+                        pp[4 * u] = w.x, pp[4 * u + 1] = w.y, pp[4 * u + 2] = w.z, pp[4 * u + 3] = w.w;
+                    }
+#pragma unroll
+                    for (int u = 0; u < 16; ++u) {
+                        const float with = acc + pp[u] * vv[u];
+                        acc = pp[u] != 0.f ? with : acc;      // a key of weight zero (masked, or past the end) adds nothing, whatever V holds
+                    }
+                };
+                for (int k0 = 0; k0 < valid; k0 += 16) add_keys(k0);
+            }
+            if (b + 1 < blocks) put_v((b + 1) & 1);
+            __syncthreads();
+        }
+    }
+    if (tid >= v_dim) return;
+    float inv = l_run > 0.f ? 1.f / l_run : 0.f;
+    if (head_gate) inv *= head_gate[t * num_q_heads + h];
+    out[t * out_stride + (int64_t)h * v_dim + tid] = from_float<T>(acc * inv);
+}
+
 template <int N> struct Count { static constexpr int value = N; };
 
 #define ATT_ROWS 32              // query rows of a workgroup of the tiled kernel
@@ -510,6 +656,19 @@ NVA_EXPORT int NVA_NAME(nva_paged_attention_generic)(
     if (page_size <= 0 || table_stride <= 0) return nva_fail("paged_attention: bad page size or table width");
     if (window < 0 || chunk < 0 || keep_first < 0) return nva_fail("paged_attention: negative window, chunk or kept positions");
     if (sig_bias && (sinks || shares > 1)) return nva_fail("paged_attention: sigmoid weights go without a sink and without shares");
+    const size_t vb = 8 * sizeof(elem_t);
+    if (shares == 1 && window == 0 && !sig_bias && head_dim <= ATT_SINGLE_MAX_D && v_dim <= ATT_SINGLE_MAX_D && head_dim % 8 == 0 &&
+        page_size % 32 == 0 && nva_aligned(k_cache, vb) && nva_aligned(v_cache, vb) && tokens * num_q_heads <= ATT_SINGLE_PAIRS) {
+        const auto kernel = paged_attention_single_kernel<elem_t>;
+        constexpr int lds = 2 * ATT_SINGLE_MAX_D * ATT_V_LD * (int)sizeof(float);
+        if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
+            return nva_fail("paged_attention: %d bytes of LDS are not to be had", lds);
+        hipLaunchKernelGGL(kernel, dim3((unsigned)tokens, (unsigned)num_q_heads), dim3(ATT_SINGLE_WAVES * NVA_WAVE), lds, stream, (const elem_t*)q,
+                           q_stride, (elem_t*)out, out_stride, (const elem_t*)k_cache, (const elem_t*)v_cache, block_tables, table_stride,
+                           token_seq, positions, num_q_heads, num_kv_heads, head_dim, v_dim, page_size, scale, chunk, softcap, sinks,
+                           head_gate, error_flag);
+        return nva_check_launch("paged_attention_generic");
+    }
     dim3 grid((unsigned)tokens, (unsigned)num_q_heads, (unsigned)shares);
     hipLaunchKernelGGL(paged_attention_generic_kernel<elem_t>, grid, dim3(NVA_WAVE), 0, stream, (const elem_t*)q,
                        q_stride, (elem_t*)out, out_stride, (const elem_t*)k_cache, (const elem_t*)v_cache,
