@@ -141,6 +141,186 @@ qk_rownorm_store_kernel(const T* __restrict__ qkv, int64_t stride, PartialInput 
     }
 }
 
+#if defined(NVA_BF16)
+// ---------------------------------------------------------------------------- many tokens
+// The same for steps of many tokens whose row is there as elements: a wave a token, 16 bytes a lane and load (a head is 1
+// to 64 neighbouring lanes of eight entries, its sum and its rotation's partners a few lane exchanges away; a norm over the
+// whole projection reads the row twice, the second time from the cache), no barrier but one; a workgroup's eight tokens hand their values over through LDS, so that eight keys
+// of a channel are one store where the tokens' slots follow each other.  Rows of 4096 entries, us with one workgroup a token
+// and scalar accesses / here: 2048 tokens with rotated heads 33.5 / 17.7, with normed and mixed values 43 / 19.5; 1556 with
+// head norms 31 / 23; 2957 with whole-row norms 44.6 / 27.4 (25 MB in and out at 2048 tokens are 5 us: what is left are the
+// chains of a wave, its row's pieces and tables one after the other).  Only bfloat16: the 32-bit path's sums keep one order at every number of tokens.
+#define QKR_TOKENS 8
+#define QKR_MANY 64              // tokens from which on this form runs
+struct QkRows {
+    const __bf16* qkv; int64_t stride; __bf16* q_out; int64_t q_stride; int64_t tokens;
+    int num_heads, num_kv_heads, head_dim, v_dim;
+    const void *q_weight, *k_weight; int w_is_f32; float eps;
+    const int32_t* positions; float temp_coef; int temp_every;
+    const float* rot_table; int rot; const int32_t* slots; __bf16 *k_cache, *v_cache; int page_size, per_head, rot_interleaved, v_norm;
+    const float *v_first_in, *v_mix; float* v_first_out; int norm_unit, gates; float* gate_out;
+};
+
+__global__ void __launch_bounds__(QKR_TOKENS * NVA_WAVE)
+qk_rownorm_rows_kernel(const QkRows a) {
+    extern __shared__ __attribute__((aligned(16))) __bf16 qkr_v[];          // [QKR_TOKENS][vd]
+    __shared__ int slot_s[QKR_TOKENS];
+    const int wave = threadIdx.x / NVA_WAVE, lane = threadIdx.x % NVA_WAVE;
+    const int qd = a.num_heads * a.head_dim, kd = a.num_kv_heads * a.head_dim, vd = a.num_kv_heads * a.v_dim, width = qd + kd + vd;
+    const int lph = a.head_dim / 8, lpv = a.v_dim / 8, half = a.rot / 2;
+    const float lam = a.v_first_in ? a.v_mix[0] : 0.f;
+    const bool stores = a.k_cache != nullptr && kd > 0;
+    const int place = wave;
+    const int64_t t = (int64_t)blockIdx.x * QKR_TOKENS + place;
+    if (t >= a.tokens) {
+        if (lane == 0) slot_s[place] = -1;
+    } else {
+        const int slot = stores ? a.slots[t] : -1;
+        if (lane == 0) slot_s[place] = slot;
+        const __bf16* row = a.qkv + t * a.stride;
+        for (int i = lane; i < a.gates; i += NVA_WAVE) a.gate_out[t * a.gates + i] = 1.f / (1.f + expf(-to_float(row[width + i])));
+        float q_scale = 1.f, k_scale = 1.f;
+        if (!a.per_head && a.q_weight) {
+            float sq = 0.f, sk = 0.f;
+#pragma unroll 4
+            for (int i = lane * 8; i < qd + kd; i += NVA_WAVE * 8) {
+                float ss = 0.f, v[8];
+                load8(row + i, v);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
+                if (i < qd) sq += ss; else sk += ss;
+            }
+            q_scale = rsqrtf(wave_sum(sq) / (float)qd + a.eps);
+            k_scale = rsqrtf(wave_sum(sk) / (float)max(kd, 1) + a.eps);
+        }
+        if (a.temp_coef != 0.f) q_scale *= 1.f + a.temp_coef * logf((float)((a.positions[t] + 1) / a.temp_every) + 1.f);
+        const float* rot_row = a.rot_table ? a.rot_table + t * (int64_t)a.rot : nullptr;
+        const int page = slot >= 0 ? slot / a.page_size : 0, off = slot >= 0 ? slot % a.page_size : 0;
+        typedef __attribute__((ext_vector_type(8))) __bf16 v8;
+        constexpr int AHEAD = 4;                           // pieces of the row that are on their way
+        v8 next[AHEAD];
+#pragma unroll
+        for (int j = 0; j < AHEAD; ++j) next[j] = *reinterpret_cast<const v8*>(row + min((j * NVA_WAVE + lane) * 8, width - 8));
+        for (int i0 = 0; i0 < width; i0 += NVA_WAVE * 8) {
+            const int i = i0 + lane * 8;
+            float x[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = (float)next[0][e];
+#pragma unroll
+            for (int j = 0; j + 1 < AHEAD; ++j) next[j] = next[j + 1];
+            next[AHEAD - 1] = *reinterpret_cast<const v8*>(row + min(i + AHEAD * NVA_WAVE * 8, width - 8));
+            const bool is_q = i < qd, is_v = i >= qd + kd;
+            // (the exchanges between lanes below are for all of them: heads lie in whole groups of lph or lpv lanes)
+            float ss = 0.f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) ss += x[e] * x[e];
+            if (a.per_head || a.v_norm)
+                for (int o = 1; o < max(lph, lpv); o <<= 1) {
+                    const float other = __shfl_xor(ss, o, NVA_WAVE);
+                    if (o < (is_v ? lpv : lph)) ss += other;
+                }
+            if (!is_v) {
+                float scale = is_q ? q_scale : k_scale;
+                const void* w = is_q ? a.q_weight : a.k_weight;
+                const int at = is_q ? i : i - qd, d = at % a.head_dim;
+                if (a.per_head && (w || a.norm_unit)) scale *= rsqrtf(ss / (float)a.head_dim + a.eps);
+                float wv[8];
+                if (w) {
+                    const int wi = a.per_head ? d : at;
+                    if (a.w_is_f32) load8(static_cast<const float*>(w) + wi, wv); else load8(static_cast<const __bf16*>(w) + wi, wv);
+                }
+#pragma unroll
+                for (int e = 0; e < 8; ++e) x[e] *= w ? scale * wv[e] : scale;
+            }
+            if (rot_row) {
+                const int d = (is_q ? i : i - qd) % a.head_dim;
+                const bool turned = !is_v && d < a.rot;
+                if (a.rot_interleaved) {
+                    if (turned) {
+                        const float4 c = *reinterpret_cast<const float4*>(rot_row + d / 2), sn = *reinterpret_cast<const float4*>(rot_row + half + d / 2);
+                        const float cs[4] = {c.x, c.y, c.z, c.w}, sns[4] = {sn.x, sn.y, sn.z, sn.w};
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const float u = x[2 * e], v = x[2 * e + 1];
+                            x[2 * e] = u * cs[e] - v * sns[e];
+                            x[2 * e + 1] = v * cs[e] + u * sns[e];
+                        }
+                    }
+                } else {
+                    float other[8];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) other[e] = __shfl_xor(x[e], half / 8, NVA_WAVE);
+                    if (turned) {
+                        const bool low = d < half;
+                        float c[8], sn[8];
+                        load8(rot_row + (low ? d : d - half), c);
+                        load8(rot_row + half + (low ? d : d - half), sn);
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) x[e] = low ? x[e] * c[e] - other[e] * sn[e] : x[e] * c[e] + other[e] * sn[e];
+                    }
+                }
+            }
+            if (i >= width) continue;
+            if (is_q) {
+                store8(a.q_out + t * a.q_stride + i, x);
+            } else if (!is_v) {
+                const int at = i - qd, g = at / a.head_dim;
+                if (slot >= 0) store8(a.k_cache + (((int64_t)page * a.num_kv_heads + g) * a.page_size + off) * a.head_dim + at % a.head_dim, x);
+            } else {
+                const int at = i - qd - kd;
+                if (a.v_norm) {
+                    const float scale = rsqrtf(ss / (float)a.v_dim + a.eps);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) x[e] *= scale;
+                }
+                if (a.v_first_out) store8(a.v_first_out + t * vd + at, x);
+                if (a.v_first_in) {
+                    float v[8];
+                    load8(a.v_first_in + t * vd + at, v);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) x[e] = (1.f - lam) * x[e] + lam * v[e];
+                }
+                if (stores) store8(qkr_v + place * vd + at, x);
+            }
+        }
+    }
+    if (!stores) return;
+    __syncthreads();
+    const int vt = nva_v_tile(a.page_size), slot0 = slot_s[0];
+    bool run = slot0 >= 0 && slot0 % QKR_TOKENS == 0 && a.page_size % QKR_TOKENS == 0 && vt % QKR_TOKENS == 0;
+#pragma unroll
+    for (int j = 1; j < QKR_TOKENS; ++j) run = run && slot_s[j] == slot0 + j;
+    for (int c = threadIdx.x; c < vd; c += QKR_TOKENS * NVA_WAVE) {
+        const int g = c / a.v_dim, d = c % a.v_dim;
+        typedef __attribute__((ext_vector_type(8))) __bf16 v8;
+        v8 v;
+#pragma unroll
+        for (int j = 0; j < QKR_TOKENS; ++j) v[j] = qkr_v[j * vd + c];
+        auto at = [&](int slot) -> __bf16* {
+            return a.v_cache + ((int64_t)(slot / a.page_size) * a.num_kv_heads + g) * a.v_dim * (int64_t)a.page_size +
+                   nva_v_offset(slot % a.page_size, d, a.v_dim, vt);
+        };
+        if (run) *reinterpret_cast<v8*>(at(slot0)) = v;
+        else
+#pragma unroll
+            for (int j = 0; j < QKR_TOKENS; ++j)
+                if (slot_s[j] >= 0) *at(slot_s[j]) = v[j];
+    }
+}
+
+// Whether the form for many tokens takes these sizes, strides and addresses.
+static bool qkr_takes(const QkRows& a) {
+    const auto pow2 = [](int n) { return n > 0 && (n & (n - 1)) == 0; };
+    const int qd = a.num_heads * a.head_dim, kd = a.num_kv_heads * a.head_dim, vd = a.num_kv_heads * a.v_dim;
+    const size_t wb = a.w_is_f32 ? 32 : 16;
+    return a.tokens >= QKR_MANY && a.head_dim % 8 == 0 && a.v_dim % 8 == 0 && pow2(a.head_dim / 8) && pow2(a.v_dim / 8) && a.head_dim <= 512 &&
+           a.v_dim <= 512 && (qd + kd) % a.v_dim == 0 && a.stride % 8 == 0 && a.q_stride % 8 == 0 &&
+           nva_aligned(a.qkv, 16) && nva_aligned(a.q_out, 16) && nva_aligned(a.q_weight, wb) && nva_aligned(a.k_weight, wb) &&
+           nva_aligned(a.k_cache, 16) && nva_aligned(a.v_cache, 16) && nva_aligned(a.v_first_in, 32) && nva_aligned(a.v_first_out, 32) &&
+           (!a.rot_table || (nva_aligned(a.rot_table, 32) && a.rot % 16 == 0 && (a.rot_interleaved || pow2(a.rot / 16))));
+}
+#endif
+
 // qkv: [tokens, Hq * D + Hkv * D + Hkv * DV] with rows `stride` elements apart, or (sums != null) the float
 // partial sums [splits][tokens][width] of the projection with its bias, which are added up here.
 // row_width: the columns of a row of the projection, gate columns and padding included.
@@ -180,6 +360,17 @@ NVA_EXPORT int NVA_NAME(nva_qk_rownorm_store)(const void* qkv, int64_t stride, c
     if (v_first_in && (!v_mix || v_first_out)) return nva_fail("qk_rownorm_store: mixing values needs the factor, and reads or writes the first values, not both");
     if ((k_cache || v_cache) && (!k_cache || !v_cache || !slots || page_size <= 0 || !num_kv_heads))
         return nva_fail("qk_rownorm_store: storing needs both caches, the slots and the page size");
+#if defined(NVA_BF16)
+    const QkRows rows{(const __bf16*)qkv, stride, (__bf16*)q_out, q_stride, tokens, num_heads, num_kv_heads, head_dim, v_dim, q_weight, k_weight,
+                      w_is_f32, eps, positions, temp_coef, temp_every, rot_table, rot_table ? rot : 0, slots, (__bf16*)k_cache, (__bf16*)v_cache,
+                      page_size, per_head ? 1 : 0, rot_interleaved ? 1 : 0, v_norm ? 1 : 0, v_first_in, v_mix, v_first_out, norm_unit ? 1 : 0,
+                      gates, gate_out};
+    const size_t rows_lds = (size_t)QKR_TOKENS * num_kv_heads * v_dim * sizeof(__bf16);
+    if (!sums && rows_lds <= 48 * 1024 && qkr_takes(rows)) {
+        hipLaunchKernelGGL(qk_rownorm_rows_kernel, dim3((unsigned)((tokens + QKR_TOKENS - 1) / QKR_TOKENS)), dim3(QKR_TOKENS * NVA_WAVE), rows_lds, stream, rows);
+        return nva_check_launch("qk_rownorm_store");
+    }
+#endif
     auto kernel = qk_rownorm_store_kernel<elem_t>;
     const size_t lds = (size_t)(width + (per_head ? num_heads + num_kv_heads : 0) + (v_norm ? num_kv_heads : 0)) * sizeof(float);
     static bool raised = false;
