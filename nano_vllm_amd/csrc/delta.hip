@@ -18,8 +18,8 @@
 //
 // Everything after the projections is float whatever the element type (the convolutions' sums, the unit norms,
 // softplus and the exponentials by the accurate routines, the state, the read-out, the norm and the gate); y is
-// rounded once.  A token's sums run in an order that neither the portion's cut nor the batch changes: the
-// recurrence goes token by token, 8 or 16 lanes holding one column of S in registers.
+// rounded once.  Outside the blocks below a token's sums run in an order that neither the portion's cut nor the batch
+// changes: the recurrence goes token by token, 8 or 16 lanes holding one column of S in registers.
 //
 //   delta_prepare     one workgroup per (token, head of q, k or v): the convolutions, unit norms, beta and the decay,
 //                     written as floats
@@ -29,8 +29,9 @@
 //                     v asked for a batch ahead
 //   delta_finish      one wave per (token, head): the norm and the gate
 //
-// With one decay per head two more ways run the same rule:
-//   delta_single      a request that brings one token: everything above for one (request, value head) in one workgroup
+// Two more ways run the same rule:
+//   delta_single      with one decay per head, a request that brings one token: everything above for one (request, value
+//                     head) in one workgroup
 //   delta_block_*     portions of many tokens, in blocks of 64 on the matrix cores (float products).  With G_i the sum of
 //                     the logarithms of the decays up to token i of a block, S_0 the state before the block, and
 //                     A_ij = beta_i exp(G_i - G_j) k_i.k_j for j < i, the writes of the block are
@@ -42,6 +43,8 @@
 //     delta_block_solve     a workgroup per (block, head): A and P by products; U and W by substitution in blocks of 16 rows,
 //                           the diagonal blocks of I + A inverted row by row, everything else products
 //     delta_block_scan      a workgroup per (portion, head, 16 columns of S): the blocks one after the other
+//                     With a decay per channel (bfloat16 models only) exp(G_i - G_j) stands inside the sums over the channels,
+//                     as the product of the decays between: see delta_block_solve.
 #include "common.h"
 
 typedef __attribute__((ext_vector_type(4))) float delta_f32x4;
@@ -471,9 +474,10 @@ delta_single_kernel(const T* __restrict__ proj, int64_t stride, DeltaRates rates
 // [KB x 16 channels], p [ub][4 x 16 tokens][4 x 16 tokens], k_t [ub][KB x 16 channels][4 x 16 tokens], all as left operands
 // (row lane % 16, columns 4 (lane / 16) + j), u [ub][DV / 16][4 x 16 tokens] as results (rows 4 (lane / 16) + i, column
 // lane % 16).  Tokens past a block's end are zeros in w, p, k_t and u.
-template <typename T, int TAPS>
+template <typename T, int TAPS, bool HEAD>
 __global__ void __launch_bounds__(DELTA_PREPARE_THREADS)
-delta_block_prepare_kernel(const T* __restrict__ proj, int64_t stride, DeltaRates rates, const T* __restrict__ conv_w,
+delta_block_prepare_kernel(const T* __restrict__ proj, int64_t stride, DeltaRates rates, const float* __restrict__ decay_in,
+                           const T* __restrict__ conv_w,
                            const float* __restrict__ dt_bias, const float* __restrict__ a_log,
                            const float* __restrict__ conv_state, const int32_t* __restrict__ units,
                            const int32_t* __restrict__ cu_seqlens_q, const int32_t* __restrict__ seq_starts,
@@ -561,6 +565,22 @@ delta_block_prepare_kernel(const T* __restrict__ proj, int64_t stride, DeltaRate
         for (int i = 0; i < N; ++i)
             if (i < nt) vf[(tok0 + i) * vv + h * vdim + d] = y[i];
     }
+    if (!HEAD) {
+        // a decay per key channel (in the padding, where q and k are zeros: ones)
+        const float rate = expf(a_log[h]);
+        for (int d = tid; d < dp; d += DELTA_PREPARE_THREADS) {
+            const int c = h * dim + min(d, dim - 1);
+            const float bias = dt_bias[c];
+            float z[N];
+#pragma unroll
+            for (int i = 0; i < N; ++i) z[i] = decay_in[(tok0 + min(i, nt - 1)) * (int64_t)(heads * dim) + c];
+#pragma unroll
+            for (int i = 0; i < N; ++i)
+                if (i < nt) decay[((tok0 + i) * heads + h) * dp + d] = d < dim ? expf(-rate * delta_softplus(z[i] + bias)) : 1.f;
+        }
+        if (tid < nt) beta[(tok0 + tid) * heads + h] = 1.f / (1.f + expf(-to_float(proj[(tok0 + tid) * stride + channels + h])));
+        return;
+    }
     if (tid < nt) {
         decay[(tok0 + tid) * heads + h] = -expf(a_log[h]) * delta_softplus(delta_rate(rates, tok0 + tid, heads, heads + h) + dt_bias[h]);
         beta[(tok0 + tid) * heads + h] = 1.f / (1.f + expf(-delta_rate(rates, tok0 + tid, heads, h)));
@@ -570,8 +590,38 @@ delta_block_prepare_kernel(const T* __restrict__ proj, int64_t stride, DeltaRate
 // KB: steps of 16 key channels (dim <= 16 KB).  Products by v_mfma_f32_16x16x4_f32: lane l holds row (or column) l % 16 and,
 // over the four instructions of a step of 16 channels, the channels 4 (l / 16) + j of both operands; results: row
 // 4 (l / 16) + i, column l % 16.
-template <int KB>
-__global__ void __launch_bounds__(256)
+//
+// HEAD false: decays a_t per key channel.  g_cum then receives each channel's product over the block, [ub][16 KB], and q is
+// left multiplied by the products up to its token.  The entry of k k^T or q k^T between the tokens r and c is a sum over the
+// channels of k_r k_c a_(c+1) ... a_r: a 16 x 16 block below the diagonal splits each product at the start of its rows, which
+// leaves a factor of the row and one of the column.  On the diagonal the split has to differ by entry: halves of 16, 8, 4 and
+// 2 tokens, a product of matrices each, whose entry is taken where row and column part at that half.  Every factor is a
+// product of decays of tokens between c and r alone: nothing is divided and nothing exceeds one, whatever the decays (sums of
+// logarithms lose the digits of a decay before both tokens, and cost an exponential a factor).
+// Bound by the serial steps within a block (its products, its inverse, the substitution): two workgroups a compute unit, hence
+// the limit on registers.  32 heads of 128 x 128, portions of 541, 610 and 405 tokens: 72 us, 108 with one workgroup.  With
+// the preparation (45) and the pass over the blocks (64, the matrix cores' time at 32 bits is 40) 181 us; token by token 280.
+
+// Inclusive products along the 16 lanes of a row from its start, and, exclusive of the lane, to its end.
+template <int CTRL>
+__device__ __forceinline__ float delta_lane(float x) {                  // the lane's that many on, one past the row's ends
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0x3f800000, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, false));
+}
+__device__ __forceinline__ float delta_products_before(float x) {
+    x *= delta_lane<0x111>(x);
+    x *= delta_lane<0x112>(x);
+    x *= delta_lane<0x114>(x);
+    return x * delta_lane<0x118>(x);
+}
+__device__ __forceinline__ float delta_products_after(float x) {
+    x = delta_lane<0x101>(x);
+    x *= delta_lane<0x101>(x);
+    x *= delta_lane<0x102>(x);
+    x *= delta_lane<0x104>(x);
+    return x * delta_lane<0x108>(x);
+}
+template <int KB, bool HEAD>
+__global__ void __launch_bounds__(256, HEAD ? 1 : 2)
 delta_block_solve_kernel(const float* __restrict__ qn, const float* __restrict__ kn, const float* __restrict__ vf,
                          const float* __restrict__ decay, const float* __restrict__ beta, const int32_t* __restrict__ units,
                          int heads, int kv_heads, int dim, int vdim, float* __restrict__ g_cum, delta_f32x4* __restrict__ w_out,
@@ -589,7 +639,24 @@ delta_block_solve_kernel(const float* __restrict__ qn, const float* __restrict__
     const int kvh = h / (heads / kv_heads);
     const int dp = (dim + 3) & ~3, vv = heads * vdim;
     const int tid = threadIdx.x, wave = tid / NVA_WAVE, lane = tid % NVA_WAVE, col = lane & 15, g = lane >> 4;
-    if (wave == 0) {
+    constexpr int W = 16 * KB;
+    __shared__ __attribute__((aligned(16))) float t_s[HEAD ? 1 : 4][HEAD ? 4 : W];     // 16 tokens' products of decays, by channel
+    if (!HEAD) {
+        for (int i = tid; i < 4 * W; i += 256) {
+            const int b = i / W, d = i % W;
+            float product = 1.f;
+#pragma unroll
+            for (int t = 16 * b; t < 16 * b + 16; ++t) {
+                const float v = decay[((first + min(t, n - 1)) * heads + h) * dp + min(d, dp - 1)];
+                product *= t < n && d < dp ? v : 1.f;
+            }
+            t_s[HEAD ? 0 : b][HEAD ? 0 : d] = product;
+        }
+        if (tid < DELTA_BLOCK) b_s[tid] = tid < n ? beta[(first + tid) * heads + h] : 0.f;
+        __syncthreads();
+        if (tid < W) g_cum[ub * W + tid] = ((t_s[0][tid] * t_s[HEAD ? 0 : 1][tid]) * t_s[HEAD ? 0 : 2][tid]) * t_s[HEAD ? 0 : 3][tid];
+    }
+    if (HEAD && wave == 0) {
         float sum = lane < n ? decay[(first + lane) * heads + h] : 0.f;
 #pragma unroll
         for (int off = 1; off < NVA_WAVE; off <<= 1) {
@@ -611,6 +678,86 @@ delta_block_solve_kernel(const float* __restrict__ qn, const float* __restrict__
         return *reinterpret_cast<const delta_f32x4*>(&tile_s[wave][col][4 * g]);
     };
     // the ten blocks of 16 x 16 on and below the diagonal, of k k^T and of q k^T
+    if constexpr (!HEAD) {
+        const float* lrow = decay + first * heads * dp + h * dp + 4 * g;
+        for (int pair = wave; pair < 10; pair += 4) {
+            const int o = pair - 4, bi = pair < 4 ? pair : o < 1 ? 1 : o < 3 ? 2 : 3, bj = pair < 4 ? pair : o - bi * (bi - 1) / 2;    // the diagonal first
+            const int ra = 16 * bi + col, rb = 16 * bj + col;
+            const int64_t at_a = ((first + min(ra, n - 1)) * kv_heads + kvh) * dp + 4 * g, at_b = ((first + min(rb, n - 1)) * kv_heads + kvh) * dp + 4 * g;
+            const int64_t la = (int64_t)min(ra, n - 1) * heads * dp, lb = (int64_t)min(rb, n - 1) * heads * dp;
+            const delta_f32x4 zero = {0.f, 0.f, 0.f, 0.f}, one = {1.f, 1.f, 1.f, 1.f};
+            delta_f32x4 ak = zero, aq = zero;
+            if (bi != bj) {
+#pragma unroll 2
+                for (int s = 0; s < KB; ++s) {
+                    const int d = 16 * s + 4 * g;
+                    delta_f32x4 fq = zero, fk = zero, fb = zero, ga = one, gb = one;
+                    if (d < dp) {
+                        fq = *reinterpret_cast<const delta_f32x4*>(qn + at_a + 16 * s);
+                        fk = *reinterpret_cast<const delta_f32x4*>(kn + at_a + 16 * s);
+                        fb = *reinterpret_cast<const delta_f32x4*>(kn + at_b + 16 * s);
+                        if (ra < n) ga = *reinterpret_cast<const delta_f32x4*>(lrow + la + 16 * s);
+                        if (rb < n) gb = *reinterpret_cast<const delta_f32x4*>(lrow + lb + 16 * s);
+                    }
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float ea = delta_products_before(ga[e]);
+                        float eb = delta_products_after(gb[e]) * fb[e];
+                        for (int b = bj + 1; b < bi; ++b) eb *= t_s[b][d + e];
+                        ak = __builtin_amdgcn_mfma_f32_16x16x4f32(fk[e] * ea, eb, ak, 0, 0, 0);
+                        aq = __builtin_amdgcn_mfma_f32_16x16x4f32(fq[e] * ea, eb, aq, 0, 0, 0);
+                    }
+                }
+            } else {
+                delta_f32x4 hk[4] = {zero, zero, zero, zero}, hq[4] = {zero, zero, zero, zero};
+#pragma unroll 2
+                for (int s = 0; s < KB; ++s) {
+                    const int d = 16 * s + 4 * g;
+                    delta_f32x4 fq = zero, fk = zero, ga = one, v;
+                    if (d < dp) {
+                        fq = *reinterpret_cast<const delta_f32x4*>(qn + at_a + 16 * s);
+                        fk = *reinterpret_cast<const delta_f32x4*>(kn + at_a + 16 * s);
+                        if (ra < n) ga = *reinterpret_cast<const delta_f32x4*>(lrow + la + 16 * s);
+                    }
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        ak = __builtin_amdgcn_mfma_f32_16x16x4f32(fk[e], fk[e], ak, 0, 0, 0);
+                        aq = __builtin_amdgcn_mfma_f32_16x16x4f32(fq[e], fk[e], aq, 0, 0, 0);
+                        float before = ga[e], after = 1.f;              // products within the runs of 1, 2, 4, 8 tokens
+                        auto step = [&](int l, float other) __attribute__((always_inline)) {       // other: the run beside, whole
+                            const float eb = after * fk[e];
+                            hk[l] = __builtin_amdgcn_mfma_f32_16x16x4f32(fk[e] * before, eb, hk[l], 0, 0, 0);
+                            hq[l] = __builtin_amdgcn_mfma_f32_16x16x4f32(fq[e] * before, eb, hq[l], 0, 0, 0);
+                            if (col & (1 << l)) before *= other; else after *= other;
+                        };
+                        step(0, delta_lane<0xb1>(before));               // the lane's neighbour, its pair's, its four's, its eight's
+                        step(1, delta_lane<0x4e>(before * after));
+                        step(2, delta_lane<0x141>(before * after));
+                        step(3, delta_lane<0x140>(before * after));
+                        for (int b = 0; b < bi; ++b) before *= t_s[b][d + e];
+                        v[e] = fq[e] * before;
+                    }
+                    q_out[((ub * 4 + bi) * KB + s) * NVA_WAVE + lane] = v;
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int part = (4 * g + i) ^ col;
+                    if (part) {
+                        ak[i] = part >= 8 ? hk[3][i] : part >= 4 ? hk[2][i] : part >= 2 ? hk[1][i] : hk[0][i];
+                        aq[i] = part >= 8 ? hq[3][i] : part >= 4 ? hq[2][i] : part >= 2 ? hq[1][i] : hq[0][i];
+                    }
+                }
+            }
+            delta_f32x4 v;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int r = 16 * bi + 4 * g + i, c = 16 * bj + col;
+                a_s[r][c] = r < n && c < r ? b_s[r] * ak[i] : 0.f;
+                v[i] = r < n && c <= r ? aq[i] : 0.f;
+            }
+            p_out[((ub * 4 + bi) * 4 + bj) * NVA_WAVE + lane] = turned(v);
+        }
+    } else
     for (int task = wave; task < 20; task += 4) {
         const int pair = task >> 1;
         const bool of_q = task & 1;
@@ -690,13 +837,53 @@ delta_block_solve_kernel(const float* __restrict__ qn, const float* __restrict__
         const int d = 16 * (of_v ? cb : cb - v_blocks) + col, width = of_v ? vdim : dp;
         const float* src = of_v ? vf + first * vv + h * vdim : kn + (first * kv_heads + kvh) * dp;
         const int64_t step = of_v ? vv : (int64_t)kv_heads * dp;
-        const float* scale = of_v ? b_s : bg_s;                         // (zero past the block's end)
+        const float* scale = of_v || !HEAD ? b_s : bg_s;                // (zero past the block's end)
         delta_f32x4 x[4];
 #pragma unroll
         for (int bi = 0; bi < 4; ++bi)
 #pragma unroll
             for (int i = 0; i < 4; ++i) x[bi][i] = src[min(16 * bi + 4 * g + i, n - 1) * step + min(d, width - 1)];
-        if (!of_v) {
+        delta_f32x4 since[HEAD ? 1 : 4];                                // the channel's product up to each token, for W
+        if constexpr (!HEAD) {
+            if (!of_v) {
+                float total[4], before = 1.f;
+                delta_f32x4 l[4];
+#pragma unroll
+                for (int bi = 0; bi < 4; ++bi) {
+                    total[bi] = t_s[bi][d];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const int t = 16 * bi + 4 * g + i;
+                        const float v = decay[((first + min(t, n - 1)) * heads + h) * dp + min(d, dp - 1)];
+                        l[bi][i] = t < n && d < dp ? v : 1.f;
+                    }
+                }
+#pragma unroll
+                for (int bi = 0; bi < 4; ++bi) {
+                    const float own = (l[bi][0] * l[bi][1]) * (l[bi][2] * l[bi][3]);
+                    float up = before, down = 1.f;
+#pragma unroll
+                    for (int b = bi + 1; b < 4; ++b) down *= total[b];
+#pragma unroll
+                    for (int o = 0; o < 4; ++o) {                       // the other lanes' fours of the 16 tokens
+                        const float other = __shfl(own, col + 16 * o, NVA_WAVE);
+                        up *= o < g ? other : 1.f;
+                        down *= o > g ? other : 1.f;
+                    }
+                    delta_f32x4 v;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) since[bi][i] = up *= l[bi][i];
+#pragma unroll
+                    for (int i = 3; i >= 0; --i) {
+                        v[i] = 16 * bi + 4 * g + i < n ? x[bi][i] * down : 0.f;
+                        down *= l[bi][i];
+                    }
+                    kt_out[((ub * KB + cb - v_blocks) * 4 + bi) * NVA_WAVE + lane] = v;
+                    before *= total[bi];
+                }
+            }
+        }
+        if (HEAD && !of_v) {
 #pragma unroll
             for (int bi = 0; bi < 4; ++bi) {
                 delta_f32x4 v;
@@ -712,7 +899,11 @@ delta_block_solve_kernel(const float* __restrict__ qn, const float* __restrict__
         for (int bi = 0; bi < 4; ++bi) {
             delta_f32x4 r;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) r[i] = x[bi][i] * scale[16 * bi + 4 * g + i];
+            for (int i = 0; i < 4; ++i) {
+                const int t = 16 * bi + 4 * g + i;
+                r[i] = x[bi][i] * scale[t];
+                if (!HEAD && !of_v) r[i] *= since[HEAD ? 0 : bi][i];
+            }
 #pragma unroll
             for (int bj = 0; bj < bi; ++bj)
 #pragma unroll
@@ -736,7 +927,8 @@ __device__ __forceinline__ void delta_barrier() { asm volatile("s_waitcnt lgkmcn
 // chains: int32 [n][4] = (a portion's first block, its blocks, its request, unused).  One workgroup of four waves per (head,
 // portion, 16 columns of S), heads fastest, so that the workgroups of a head meet in one die's L2.  The state's columns lie
 // in accumulators (wave w: the blocks w, w + 4, ... of 16 rows) and, transposed, in LDS for the products that read them.
-template <int KB>
+// HEAD false: g_cum holds a channel's product of decays over the block, [ub][16 KB], and q comes multiplied by its decays.
+template <int KB, bool HEAD>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 delta_block_scan_kernel(const float* __restrict__ g_cum, const delta_f32x4* __restrict__ w_in, const delta_f32x4* __restrict__ q_in,
                         const delta_f32x4* __restrict__ u_in, const delta_f32x4* __restrict__ p_in,
@@ -768,7 +960,7 @@ delta_block_scan_kernel(const float* __restrict__ g_cum, const delta_f32x4* __re
     }
     // A block's operands, asked for while the block before it is at work.
     struct Operands {
-        delta_f32x4 wf[KB], qf[KB], pf[4], kt[NB][4], gi, u;
+        delta_f32x4 wf[KB], qf[KB], pf[4], kt[NB][4], gi, u, ge[NB];
         float g_end;
         int first, n;
     };
@@ -782,7 +974,7 @@ delta_block_scan_kernel(const float* __restrict__ g_cum, const delta_f32x4* __re
         const delta_f32x4* wr = w_in + (ub * 4 + wave) * KB * NVA_WAVE + lane;
         const delta_f32x4* qr = q_in + (ub * 4 + wave) * KB * NVA_WAVE + lane;
         const delta_f32x4* pr = p_in + (ub * 4 + wave) * 4 * NVA_WAVE + lane;
-        const float* gr = g_cum + ub * DELTA_BLOCK;
+        const float* gr = g_cum + ub * (HEAD ? DELTA_BLOCK : 16 * KB);
 #pragma unroll
         for (int s = 0; s < KB; ++s) {
             o.wf[s] = wr[s * NVA_WAVE];
@@ -795,8 +987,13 @@ delta_block_scan_kernel(const float* __restrict__ g_cum, const delta_f32x4* __re
         for (int b = 0; b < NB; ++b)
 #pragma unroll
             for (int s = 0; s < 4; ++s) o.kt[b][s] = kt_in[((ub * KB + min(wave + 4 * b, KB - 1)) * 4 + s) * NVA_WAVE + lane];
-        o.gi = *reinterpret_cast<const delta_f32x4*>(gr + 16 * wave + 4 * g);
-        o.g_end = gr[DELTA_BLOCK - 1];
+        if (HEAD) {
+            o.gi = *reinterpret_cast<const delta_f32x4*>(gr + 16 * wave + 4 * g);
+            o.g_end = gr[DELTA_BLOCK - 1];
+        } else {
+#pragma unroll
+            for (int b = 0; b < NB; ++b) o.ge[b] = *reinterpret_cast<const delta_f32x4*>(gr + 16 * min(wave + 4 * b, KB - 1) + 4 * g);
+        }
     };
     auto run = [&](const Operands& o) __attribute__((always_inline)) {
         // W S and Q S of this wave's 16 tokens
@@ -816,14 +1013,17 @@ delta_block_scan_kernel(const float* __restrict__ g_cum, const delta_f32x4* __re
         }
         delta_f32x4 u;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) u[i] = o.u[i] - x[i], y[i] *= expf(o.gi[i]);
+        for (int i = 0; i < 4; ++i) {
+            u[i] = o.u[i] - x[i];
+            if (HEAD) y[i] *= expf(o.gi[i]);
+        }
         *reinterpret_cast<delta_f32x4*>(&u_s[col][16 * wave + 4 * g]) = u;
         delta_barrier();                                                // the block's writes are in; the state is read
-        const float e_end = expf(o.g_end);
+        const float e_end = HEAD ? expf(o.g_end) : 0.f;
 #pragma unroll
         for (int b = 0; b < NB; ++b)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) S[b][i] *= e_end;
+            for (int i = 0; i < 4; ++i) S[b][i] *= HEAD ? e_end : o.ge[b][i];
         delta_f32x4 uv[4];
 #pragma unroll
         for (int s = 0; s < 4; ++s) uv[s] = *reinterpret_cast<const delta_f32x4*>(&u_s[col][16 * s + 4 * g]);
@@ -922,6 +1122,20 @@ static void launch_delta_keep(const void* proj, int64_t stride, float* conv_stat
 // norm_w float [DV].  conv_state float [slots, 2 G D + H DV, taps - 1], s_state float [slots, H, D, DV]: a request's
 // rows by state_slots, taken as zero where seq_starts is 0.  scratch: float [tokens * ((2 G + H) DP + 2 H DV + H)], DP = D rounded up to 4, 16-byte aligned.
 // The step's requests by cu_seqlens_q [seqs + 1]; token_seq [tokens].  out: elements [tokens, H DV].
+// units [n_units][4] and chains [n_chains][4] (see the blocks' kernels) with block_scratch (nva_channel_delta_block_floats) cover the
+// requests after the first `singles`, which bring one token each: those then run in blocks; n_units 0: token by token.
+static int delta_steps(int dim) { return dim <= 32 ? 2 : dim <= 64 ? 4 : dim <= 128 ? 8 : 16; }      // steps of 16 key channels the blocks' kernels are built for
+
+// Floats that block_scratch holds for n blocks of portions, or 0 where blocks do not take the sizes.
+NVA_EXPORT int64_t NVA_NAME(nva_channel_delta_block_floats)(int64_t n, int heads, int dim, int vdim, int taps) {
+#ifdef NVA_F32
+    return 0;                       // (32-bit models: the order of a request's sums is the same in every step)
+#endif
+    if (dim > 128 || taps > 4) return 0;
+    const int64_t w = 16 * (int64_t)delta_steps(dim);
+    return n * heads * (DELTA_BLOCK * (3 * w + (vdim + 15) / 16 * 16 + DELTA_BLOCK) + w);
+}
+
 NVA_EXPORT int NVA_NAME(nva_channel_delta)(const void* proj, int64_t stride, const float* decay_in, const void* gate_in,
                                            int64_t gate_stride, float* scratch, void* out, int64_t out_stride,
                                            float* s_state, float* conv_state, const int32_t* token_seq,
@@ -929,7 +1143,8 @@ NVA_EXPORT int NVA_NAME(nva_channel_delta)(const void* proj, int64_t stride, con
                                            const int32_t* state_slots, int64_t seqs, int64_t tokens, int heads,
                                            int kv_heads, int dim, int vdim, int taps, const void* conv_w,
                                            const float* dt_bias, const float* a_log, const float* norm_w, float eps,
-                                           hipStream_t stream) {
+                                           int64_t singles, const int32_t* units, int64_t n_units, const int32_t* chains,
+                                           int64_t n_chains, float* block_scratch, hipStream_t stream) {
     if (tokens == 0) return 0;
     const int qk = kv_heads * dim, vv = heads * vdim, channels = 2 * qk + vv;
     const int bad = check_delta("channel_delta", proj, stride, channels + (int64_t)heads, scratch, out, out_stride, s_state, conv_state,
@@ -945,13 +1160,52 @@ NVA_EXPORT int NVA_NAME(nva_channel_delta)(const void* proj, int64_t stride, con
     float* vf = decay + tokens * (int64_t)heads * dp;
     float* o_raw = vf + tokens * vv;
     float* beta = o_raw + tokens * vv;
-    hipLaunchKernelGGL((delta_prepare_kernel<elem_t, false>), dim3((unsigned)tokens, (unsigned)(2 * kv_heads + heads)),
-                       dim3(DELTA_PREPARE_THREADS), 0, stream, (const elem_t*)proj, stride, decay_in, DeltaRates{nullptr, 0, 0},
-                       (int64_t)0, (const elem_t*)conv_w, dt_bias, a_log, conv_state, token_seq, cu_seqlens_q, seq_starts, state_slots,
-                       heads, kv_heads, dim, vdim, taps, qn, kn, vf, decay, beta);
+    if (n_units && (!units || !chains || n_chains <= 0 || !block_scratch || (uintptr_t)block_scratch % 16 || n_units < n_chains || singles < 0 ||
+                    singles > seqs || !NVA_NAME(nva_channel_delta_block_floats)(n_units, heads, dim, vdim, taps) ||
+                    n_units * heads * (DELTA_BLOCK / 16) > 0x7fffffff || n_chains * heads * (int64_t)((vdim + 15) / 16) > 0x7fffffff))
+        return nva_fail("channel_delta: bad blocks (%lld in %lld portions)", (long long)n_units, (long long)n_chains);
+    const elem_t* pr = (const elem_t*)proj;
+    const elem_t* cw = (const elem_t*)conv_w;
+    const unsigned heads_y = (unsigned)(2 * kv_heads + heads);
+    const int64_t one_by_one = n_units ? singles : seqs, plain_tokens = n_units ? singles : tokens;    // requests, and their tokens
+    if (plain_tokens > 0)
+        hipLaunchKernelGGL((delta_prepare_kernel<elem_t, false>), dim3((unsigned)plain_tokens, heads_y), dim3(DELTA_PREPARE_THREADS), 0, stream,
+                           pr, stride, decay_in, DeltaRates{nullptr, 0, 0}, (int64_t)0, cw, dt_bias, a_log, conv_state, token_seq, cu_seqlens_q,
+                           seq_starts, state_slots, heads, kv_heads, dim, vdim, taps, qn, kn, vf, decay, beta);
+    if (n_units) {
+        const dim3 grid((unsigned)(n_units * (DELTA_BLOCK / 16)), heads_y);
+#define DELTA_BLOCK_PREPARE(TT)                                                                                           \
+        hipLaunchKernelGGL((delta_block_prepare_kernel<elem_t, TT, false>), grid, dim3(DELTA_PREPARE_THREADS), 0, stream, pr, stride,       \
+                           DeltaRates{nullptr, 0, 0}, decay_in, cw, dt_bias, a_log, conv_state, units, cu_seqlens_q, seq_starts, state_slots, \
+                           heads, kv_heads, dim, vdim, qn, kn, vf, decay, beta)
+        if (taps == 1) DELTA_BLOCK_PREPARE(1); else if (taps == 2) DELTA_BLOCK_PREPARE(2);
+        else if (taps == 3) DELTA_BLOCK_PREPARE(3); else DELTA_BLOCK_PREPARE(4);
+#undef DELTA_BLOCK_PREPARE
+    }
     launch_delta_keep(proj, stride, conv_state, cu_seqlens_q, seq_starts, state_slots, seqs, channels, taps, stream);
-    launch_delta_scan<false>(qn, kn, vf, decay, beta, o_raw, s_state, cu_seqlens_q, seq_starts, state_slots, seqs, heads, kv_heads, dim,
-                             vdim, stream);
+    if (one_by_one > 0)
+        launch_delta_scan<false>(qn, kn, vf, decay, beta, o_raw, s_state, cu_seqlens_q, seq_starts, state_slots, one_by_one, heads, kv_heads,
+                                 dim, vdim, stream);
+    if (n_units) {
+        const int64_t rows = n_units * heads * DELTA_BLOCK;
+        const unsigned slices = (unsigned)((vdim + 15) / 16);
+        const int steps = delta_steps(dim);
+        delta_f32x4* w = (delta_f32x4*)block_scratch;                   // (in units of four floats)
+        delta_f32x4* q = w + rows * 4 * steps;
+        delta_f32x4* kt = q + rows * 4 * steps;
+        delta_f32x4* u = kt + rows * 4 * steps;
+        delta_f32x4* p = u + rows * 4 * slices;
+        float* gc = (float*)(p + rows * (DELTA_BLOCK / 4));
+#define DELTA_BLOCKS(KK)                                                                                                  \
+        do {                                                                                                              \
+            hipLaunchKernelGGL((delta_block_solve_kernel<KK, false>), dim3((unsigned)(n_units * heads)), dim3(256), 0, stream, qn, kn, vf,    \
+                               decay, beta, units, heads, kv_heads, dim, vdim, gc, w, q, u, p, kt);                           \
+            hipLaunchKernelGGL((delta_block_scan_kernel<KK, false>), dim3((unsigned)(slices * n_chains * heads)), dim3(256), 0, stream, gc, w, \
+                               q, u, p, kt, o_raw, s_state, units, chains, (int)n_chains, seq_starts, state_slots, heads, dim, vdim); \
+        } while (0)
+        if (steps == 2) DELTA_BLOCKS(2); else if (steps == 4) DELTA_BLOCKS(4); else DELTA_BLOCKS(8);
+#undef DELTA_BLOCKS
+    }
     hipLaunchKernelGGL((delta_finish_kernel<elem_t, false>), dim3((unsigned)tokens, (unsigned)heads), dim3(NVA_WAVE), 0, stream, o_raw,
                        (const elem_t*)gate_in, gate_stride, norm_w, eps, (elem_t*)out, out_stride, heads, vdim, (int64_t)0);
     return nva_check_launch("channel_delta");
@@ -965,9 +1219,6 @@ static int delta_single_groups(int dim, int vdim) {
     const int rg = DELTA_SINGLE_THREADS >> cg;
     return rg >= 1 && (dim + rg - 1) / rg <= 16 ? cg : -1;
 }
-
-// Steps of 16 key channels that the blocks' kernels are built for.
-static int delta_steps(int dim) { return dim <= 32 ? 2 : dim <= 64 ? 4 : dim <= 128 ? 8 : 16; }
 
 // Floats that nva_head_delta's block_scratch holds for n blocks of portions.
 NVA_EXPORT int64_t NVA_NAME(nva_head_delta_block_floats)(int64_t n, int heads, int dim, int vdim) {
@@ -1038,7 +1289,7 @@ NVA_EXPORT int NVA_NAME(nva_head_delta)(const void* proj, int64_t stride, const 
         prepare(first, plain_tokens);
         const dim3 grid((unsigned)(n_units * (DELTA_BLOCK / 16)), heads_y);
 #define DELTA_BLOCK_PREPARE(TT)                                                                                           \
-        hipLaunchKernelGGL((delta_block_prepare_kernel<elem_t, TT>), grid, dim3(DELTA_PREPARE_THREADS), 0, stream, pr, stride, rt, cw, \
+        hipLaunchKernelGGL((delta_block_prepare_kernel<elem_t, TT, true>), grid, dim3(DELTA_PREPARE_THREADS), 0, stream, pr, stride, rt, (const float*)nullptr, cw, \
                            dt_bias, a_log, conv_state, units, cu_seqlens_q, seq_starts, state_slots, heads, kv_heads, dim, vdim, qn, kn, \
                            vf, decay, beta)
         if (taps == 1) DELTA_BLOCK_PREPARE(1); else if (taps == 2) DELTA_BLOCK_PREPARE(2);
@@ -1064,9 +1315,9 @@ NVA_EXPORT int NVA_NAME(nva_head_delta)(const void* proj, int64_t stride, const 
         float* gc = (float*)(p + rows * (DELTA_BLOCK / 4));
 #define DELTA_BLOCKS(KK)                                                                                                  \
         do {                                                                                                              \
-            hipLaunchKernelGGL((delta_block_solve_kernel<KK>), dim3((unsigned)(n_units * heads)), dim3(256), 0, stream, qn, kn, vf, decay, \
+            hipLaunchKernelGGL((delta_block_solve_kernel<KK, true>), dim3((unsigned)(n_units * heads)), dim3(256), 0, stream, qn, kn, vf, decay, \
                                beta, units, heads, kv_heads, dim, vdim, gc, w, q, u, p, kt);                                  \
-            hipLaunchKernelGGL((delta_block_scan_kernel<KK>), dim3((unsigned)(slices * n_chains * heads)), dim3(256), 0, stream, gc, w, q,   \
+            hipLaunchKernelGGL((delta_block_scan_kernel<KK, true>), dim3((unsigned)(slices * n_chains * heads)), dim3(256), 0, stream, gc, w, q,   \
                                u, p, kt, o_raw, s_state, units, chains, (int)n_chains, seq_starts, state_slots, heads, dim,           \
                                vdim);                                                                                     \
         } while (0)

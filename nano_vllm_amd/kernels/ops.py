@@ -376,6 +376,13 @@ class HipKernels:
         self.delta_blocks = True
         self.delta_single_kernel = True
         self.delta_block_min = DELTA_BLOCK
+        # the delta rule with a decay per channel: in blocks where the longest portion has more tokens than the first and the
+        # blocks' tokens, those in their padding too, are at most the second times the step's.  Token by token a portion takes
+        # 0.4 us a token, however few the requests; in blocks 75 us and 0.15 us a token, but 0.33 us a block of 32 heads where
+        # blocks fill the chip, which a full one earns back (32 heads of 128 x 128, token by token and in blocks: one portion
+        # of 128 tokens 64 and 84 us, 192: 92 and 92, 300: 135 and 105, 2048: 850 and 383; 8 of 700: 1338 and 1247; 16 of 80:
+        # 287 and 424; 16 of 257: 980 and 1037)
+        self.channel_block_rule = (256, 1.2)
         # False: the gated linear attention and the matrix memory run portions token by token too
         self.memory_blocks = True
         self.memory_unit_tokens = 0         # tokens of a unit of their portions, a multiple of MEMORY_CHUNK; 0: the rule
@@ -1857,12 +1864,39 @@ class HipKernels:
             raise KernelError("channel_delta: output does not match")
         dp = (dim + 3) // 4 * 4                         # rows of q, k and the decays are padded to whole float4s
         scratch = torch.empty(tokens * ((2 * kv_heads + heads) * dp + 2 * vv + heads), dtype=torch.float32, device=proj.device)
+        first = batch.num_decode
+        need = getattr(library.load("delta", self.suffix), f"nva_channel_delta_block_floats_{self.suffix}")
+        need.restype = ctypes.c_int64
+        n_units, n_chains, units, chains, block_scratch = self._delta_plan(
+            batch, first, proj.device, lambda n: int(need(c_i64(n), c_i32(heads), c_i32(dim), c_i32(vdim), c_i32(taps))),
+            *self.channel_block_rule)
         library.call("delta", _suffix(proj), "nva_channel_delta", _p(proj), c_i64(stride), _p(decay_in), _p(gate_in), c_i64(gs),
                      _p(scratch), _p(out), c_i64(os_), _p(s_state), _p(conv_state if taps > 1 else None), _p(batch.token_seq),
                      _p(batch.cu_seqlens_q), _p(batch.seq_starts), _p(batch.state_slots), c_i64(seqs), c_i64(tokens),
                      c_i32(heads), c_i32(kv_heads), c_i32(dim), c_i32(vdim), c_i32(taps), _p(conv_w), _p(dt_bias), _p(a_log),
-                     _p(norm_w), c_f32(eps), self._stream())
+                     _p(norm_w), c_f32(eps), c_i64(first), _p(units), c_i64(n_units), _p(chains), c_i64(n_chains), _p(block_scratch),
+                     self._stream())
         return out
+
+    def _delta_plan(self, batch, first: int, device, floats, least: int, slack: Optional[float] = None):
+        """The step's portions in blocks (the same cut for every layer of the step), where the longest is of more than `least`
+        tokens and the blocks' tokens are at most `slack` times the portions': (blocks, portions, units, chains, scratch).
+        floats(blocks): how many the scratch holds, 0 where blocks do not take the sizes."""
+        lens = batch.q_lens[first:]
+        if not self.delta_blocks or max(batch.q_lens) <= least or any(n != 1 for n in batch.q_lens[:first]) or not floats(1):
+            return 0, 0, None, None, None
+        if slack is not None and DELTA_BLOCK * sum((n + DELTA_BLOCK - 1) // DELTA_BLOCK for n in lens) > slack * sum(lens):
+            return 0, 0, None, None, None
+        kept = getattr(batch, "step_cache", None)
+        if kept is None:
+            kept = batch.step_cache = {}
+        plan = kept.get(("delta_blocks", first))
+        if plan is None:
+            flat_units, flat_chains = delta_blocks(batch.q_lens, first)
+            both = torch.tensor(flat_units + flat_chains, dtype=torch.int32).to(device, non_blocking=True)
+            plan = (len(flat_units) // 4, len(flat_chains) // 4, both[: len(flat_units)], both[len(flat_units):])
+            kept[("delta_blocks", first)] = plan
+        return (*plan, torch.empty(floats(plan[0]), dtype=torch.float32, device=device))
 
     def head_delta(self, proj: torch.Tensor, rates: torch.Tensor, heads: int, kv_heads: int, dim: int, vdim: int, taps: int,
                    conv_w: torch.Tensor, dt_bias: torch.Tensor, a_log: torch.Tensor, norm_w: torch.Tensor, eps: float,
@@ -1900,25 +1934,11 @@ class HipKernels:
             raise KernelError("head_delta: the first num_decode requests of a batch must bring one token each")
         dp = (dim + 3) // 4 * 4
         scratch = torch.empty(tokens * (2 * kv_heads * dp + 2 * vv + 2 * heads), dtype=torch.float32, device=proj.device)
-        # the step's portions in blocks (the same cut for every layer of the step)
-        units = chains = block_scratch = None
-        n_units = n_chains = 0
         first = batch.num_decode
-        if self.delta_blocks and max(batch.q_lens) > self.delta_block_min:
-            kept = getattr(batch, "step_cache", None)
-            if kept is None:
-                kept = batch.step_cache = {}
-            plan = kept.get(("delta_blocks", first))
-            if plan is None:
-                flat_units, flat_chains = delta_blocks(batch.q_lens, first)
-                both = torch.tensor(flat_units + flat_chains, dtype=torch.int32).to(proj.device, non_blocking=True)
-                plan = (len(flat_units) // 4, len(flat_chains) // 4, both[: len(flat_units)], both[len(flat_units):])
-                kept[("delta_blocks", first)] = plan
-            n_units, n_chains, units, chains = plan
-            need = getattr(library.load("delta", self.suffix), f"nva_head_delta_block_floats_{self.suffix}")
-            need.restype = ctypes.c_int64
-            block_scratch = torch.empty(int(need(c_i64(n_units), c_i32(heads), c_i32(dim), c_i32(vdim))), dtype=torch.float32,
-                                        device=proj.device)
+        need = getattr(library.load("delta", self.suffix), f"nva_head_delta_block_floats_{self.suffix}")
+        need.restype = ctypes.c_int64
+        n_units, n_chains, units, chains, block_scratch = self._delta_plan(
+            batch, first, proj.device, lambda n: int(need(c_i64(n), c_i32(heads), c_i32(dim), c_i32(vdim))), self.delta_block_min)
         library.call("delta", _suffix(proj), "nva_head_delta", _p(proj), c_i64(stride), _p(rate_sums), c_i32(rate_splits),
                      c_i64(tokens * 2 * heads), _p(scratch), _p(out), c_i64(os_), _p(s_state), _p(conv_state if taps > 1 else None),
                      _p(batch.token_seq), _p(batch.cu_seqlens_q), _p(batch.seq_starts), _p(batch.state_slots), c_i64(batch.num_seqs),
