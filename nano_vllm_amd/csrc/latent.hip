@@ -27,6 +27,9 @@
 //                    out of it.  A float sum over k in ascending order per output (times the head's gate, where one is
 //                    given), rounded once.
 #include "common.h"
+#include "lds_load.h"
+
+#include <type_traits>
 
 // Entry d of a turned part whose raw entries raw(0) ... raw(rot - 1) are given, by a row of rot / 2 cosines and rot / 2 sines.
 template <typename F>
@@ -428,11 +431,11 @@ NVA_EXPORT int nva_heads_linear_mfma_bf16(const void* x, int64_t x_stride, int64
 // ---------------------------------------------------------------------------- the attention itself, on the matrix cores
 // One key/value head for all query heads: the query heads of a token are the 16 columns of the products, so a key row
 // that is fetched serves all of them.  A wave takes one token, 16 of its heads and a share of its keys, in tiles of 32:
-//     S^T = K Q^T      K rows straight from the cache as the A operand (a lane 16 bytes of a key row), Q^T in registers
-//     O^T += V^T P^T   V^T from the value cache, which holds the latent transposed in tiles of 32 keys (a lane 2 x 8
-//                      bytes of a channel's row), P^T as the lanes hold it after the first product: the second
-//                      product's index over the keys is 8 g + j <-> key 4 g + j (j < 4) and 16 + 4 g + j - 4 (j >= 4)
-//                      of the tile, for both operands, so that nothing is exchanged between lanes
+//     S^T = K Q^T      K rows straight from the cache as the A operand (a lane 16 bytes of a key row), Q^T in registers;
+//                      row 4 g + i of the two products is key 8 g + i and 8 g + 4 + i of the tile
+//     O^T += V^T P^T   V^T from the value cache, which holds the latent transposed in tiles of 32 keys (a lane 16 bytes of
+//                      a channel's row), P^T as the lanes hold it after the first product, so that nothing is exchanged
+//                      between lanes
 // with an online softmax in float (exp2 with log2 e folded in), the sink as the first share's starting maximum with a
 // sum of one.  All tokens are treated alike, a prompt's and single ones (every row of a tile has the same position, so
 // only a token's last tile is masked).  With more than one share the shares leave (maximum, sum, unnormalised output)
@@ -493,12 +496,12 @@ latent_attn_kernel(const __bf16* __restrict__ q2, int64_t q_stride, __bf16* __re
             page = 0;
         }
         const int in_page = kb % page_size;
-        // ---- scores: rows of K as they lie, keys kb + col and kb + 16 + col
-        const __bf16* k0 = k_cache + ((int64_t)page * page_size + in_page + col) * width + 8 * g;
-        const __bf16* k1 = k0 + (int64_t)16 * width;
+        // ---- scores: rows of K as they lie, keys kb + 8 (col / 4) + col % 4 and four on
+        const __bf16* k0 = k_cache + ((int64_t)page * page_size + in_page + 2 * (col & 12) + (col & 3)) * width + 8 * g;
+        const __bf16* k1 = k0 + (int64_t)4 * width;
         // (all of the tile's loads are asked for before anything is used: a wave is alone on its SIMD, and what it has
         // on its way is all that hides the memory's latency)
-        const __bf16* v0 = v_cache + (((int64_t)page * tiles_per_page + in_page / LAT_TILE) * rank + col) * LAT_TILE + 4 * g;
+        const __bf16* v0 = v_cache + (((int64_t)page * tiles_per_page + in_page / LAT_TILE) * rank + col) * LAT_TILE + 8 * g;
         lat_bf16x8 ka[KS], kc[KS];
         lat_bf16x4 vlo[CB], vhi[CB];
 #pragma unroll
@@ -514,7 +517,7 @@ latent_attn_kernel(const __bf16* __restrict__ q2, int64_t q_stride, __bf16* __re
         for (int b = 0; b < CB; ++b)
             if (b < blocks) {
                 vlo[b] = *reinterpret_cast<const lat_bf16x4*>(v0 + (int64_t)b * 16 * LAT_TILE);
-                vhi[b] = *reinterpret_cast<const lat_bf16x4*>(v0 + (int64_t)b * 16 * LAT_TILE + 16);
+                vhi[b] = *reinterpret_cast<const lat_bf16x4*>(v0 + (int64_t)b * 16 * LAT_TILE + 4);
             }
         lat_f32x4 sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -524,12 +527,12 @@ latent_attn_kernel(const __bf16* __restrict__ q2, int64_t q_stride, __bf16* __re
                 sb = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kc[c], qf[c], sb, 0, 0, 0);
             }
         }
-        // this lane: head `col`, keys kb + 4 g + i (sa) and kb + 16 + 4 g + i (sb)
+        // this lane: head `col`, keys kb + 8 g + i (sa) and kb + 8 g + 4 + i (sb)
         float s[8];
         float m_new = m_run;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            const int key = kb + (i < 4 ? 4 * g + i : 16 + 4 * g + i - 4);
+            const int key = kb + 8 * g + i;
             const float raw = (i < 4 ? sa[i] : sb[i - 4]) * scale;
             s[i] = key <= pos && key >= first && !no_page ? raw : -INFINITY;
             m_new = fmaxf(m_new, s[i]);
@@ -548,7 +551,7 @@ latent_attn_kernel(const __bf16* __restrict__ q2, int64_t q_stride, __bf16* __re
         const float alpha = __builtin_amdgcn_exp2f((fmaxf(m_run, -1e30f) - m_use) * log2e);
         l_run = l_run * alpha + psum;
         m_run = m_new;
-        // ---- O^T += V^T P^T: channel 16 b + col, keys kb + 4 g .. + 3 and kb + 16 + 4 g .. + 3
+        // ---- O^T += V^T P^T: channel 16 b + col, keys kb + 8 g .. + 7
         const bool whole = kb + LAT_TILE - 1 <= pos && kb >= first && !no_page;
 #pragma unroll
         for (int b = 0; b < CB; ++b) {
@@ -559,7 +562,7 @@ latent_attn_kernel(const __bf16* __restrict__ q2, int64_t q_stride, __bf16* __re
                 if (!whole) {              // what the cache holds beyond the token's own key, or before its window, may be anything
 #pragma unroll
                     for (int e = 0; e < 8; ++e) {
-                        const int key = kb + (e < 4 ? 4 * g + e : 16 + 4 * g + e - 4);
+                        const int key = kb + 8 * g + e;
                         if (no_page || key > pos || key < first) vf[e] = (__bf16)0.f;
                     }
                 }
@@ -595,55 +598,84 @@ latent_attn_kernel(const __bf16* __restrict__ q2, int64_t q_stride, __bf16* __re
 }
 
 // The same attention for portions of prompts: a workgroup of WAVES waves (eight, or four where a latent of more than
-// 384 channels leaves a SIMD's registers to one wave) takes as many tokens in a row of one request (a part of a row tile
-// of 32 queries; tiles as for the other prefill kernels, most keys first), a wave one token.  The tiles of keys and of
-// transposed values, which the tokens share, go through LDS once for all of them:
-// the next tile is asked for (into registers) before the products of the tile at hand and stored after them.  The
-// arithmetic of a token is that of latent_attn_kernel with one share, operation for operation.
-template <int MAXC, int WAVES>
+// 384 channels leaves a SIMD's registers to one wave) takes as many tokens of one request, a wave one token (tiles of 32
+// queries as for the other prefill kernels, 32 / WAVES workgroups each).  The tiles of keys and of transposed values, which
+// the tokens share, go from the cache straight into LDS once for all of them, into one of two buffers while the products of
+// the other's tile run.  The arithmetic of a token is that of latent_attn_kernel with one share, operation for operation.
+//
+// Half of the tokens lie from the portion's start on and half before its end, counted inwards together, so that all
+// workgroups have the same number of (token, tile) pairs: 2048 tokens are 256 workgroups, one a compute unit, of which
+// the last had twice the average.  Where a window ends the keys early, a workgroup's tokens lie side by side instead, so that
+// they share their tiles.
+//
+// Bound by the reads of LDS: a wave reads the whole tile for its token, 53 KB at 448 + 384 channels, half the time at 128
+// bytes a cycle, the products beside them a quarter.  16 heads, 384 + 64 channels, 2048 tokens, 333 us before this form:
+// 167 with the pairing and loops without conditions (one at each step of 32 channels left every read of LDS to be waited for
+// by itself), 140 with reads asked for two steps ahead of their products, 113 with loads straight into LDS (more reads ahead
+// spilled while tiles passed through registers) and each lane's eight keys in a row, so that a block of values is one read
+// (8192 tokens: 2644 and 1313 us; 64 tokens behind 2000: 284 and 127; 64 alone: 20 and 14).  Two tokens a wave, which would
+// halve the reads, spill.
+template <int MAXC, int MAXR, int WAVES>
 __global__ void __launch_bounds__(WAVES * NVA_WAVE)
-latent_attn_quad_kernel(const __bf16* __restrict__ q2, int64_t q_stride, __bf16* __restrict__ out, int64_t out_stride,
+latent_attn_rows_kernel(const __bf16* __restrict__ q2, int64_t q_stride, __bf16* __restrict__ out, int64_t out_stride,
                         const __bf16* __restrict__ k_cache, const __bf16* __restrict__ v_cache,
                         const int32_t* __restrict__ block_tables, int table_stride, const int32_t* __restrict__ cu_seqlens_q,
                         const int32_t* __restrict__ kv_lens, const int32_t* __restrict__ row_tiles, int heads, int rank, int rot,
                         int page_size, float scale, int window, const float* __restrict__ sinks, int32_t* error_flag) {
-    constexpr int KS = (MAXC + LAT_MAX_ROT) / 32, CB = MAXC / 16;
-    constexpr int THREADS = WAVES * NVA_WAVE, PER_TILE = 32 / WAVES;   // tokens of a workgroup: WAVES; workgroups of a row tile
-    constexpr int KP = (4 * (MAXC + LAT_MAX_ROT) + THREADS - 1) / THREADS, VP = (4 * MAXC + THREADS - 1) / THREADS;   // 16-byte pieces of a tile a thread moves, at most
-    extern __shared__ __attribute__((aligned(16))) __bf16 lat_s[];
-    const int width = rank + rot, KSTR = width + 8, VSTR = LAT_TILE + 4;
-    __bf16* const k_s = lat_s;                          // [32 keys][KSTR]
-    __bf16* const v_s = lat_s + LAT_TILE * KSTR;        // [rank channels][VSTR]
-    const int ti = blockIdx.x / PER_TILE, quad = blockIdx.x % PER_TILE;
+    constexpr int KS = (MAXC + MAXR) / 32, CB = MAXC / 16;
+    constexpr int THREADS = WAVES * NVA_WAVE, PER_TILE = 32 / WAVES, HALF = WAVES / 2;   // workgroups of a row tile; tokens side by side
+    constexpr int KUNITS = (MAXC + MAXR) / 16, VUNITS = MAXC / 16;      // of 64 pieces of 16 bytes: a tile's keys, its values
+    constexpr int KOWN = (KUNITS + WAVES - 1) / WAVES, VOWN = (VUNITS + WAVES - 1) / WAVES;
+    constexpr int AHEAD = 3, VAHEAD = 4;                // steps that reads of LDS run before their products
+    constexpr int KROW = MAXC + MAXR, BUFFER = LAT_TILE * (KROW + MAXC);
+    extern __shared__ __attribute__((aligned(16))) __bf16 lat_s[];      // two buffers of [32 keys][KROW] and [MAXC channels][32 keys]
+    const int width = rank + rot;
+    const int ti = blockIdx.x / PER_TILE, part = blockIdx.x % PER_TILE;
     const int seq = row_tiles[2 * ti], row_tile = row_tiles[2 * ti + 1];
     const int q_begin = cu_seqlens_q[seq];
     const int q_len = cu_seqlens_q[seq + 1] - q_begin;
     const int start = kv_lens[seq] - q_len;             // position of the request's first query of this step
-    const int row0 = row_tile * 32 + quad * WAVES;
-    if (row0 >= q_len) return;                          // (the whole workgroup)
+    const int mine = row_tile * PER_TILE + part, last = (q_len + 31) / 32 * (32 / HALF) - 1;      // this workgroup, the last half
+    const bool inwards = window <= 0 || window >= start + q_len;
+    const int half_a = inwards ? mine : 2 * mine, half_b = inwards ? last - mine : 2 * mine + 1;
+    // the tiles that any token of the workgroup sees
+    int tile_0 = 0x7fffffff, tiles = 0;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int r = HALF * (i ? half_b : half_a);
+        if (r < q_len) {
+            tile_0 = min(tile_0, nva_first_key(start + r, window, 0) / LAT_TILE);
+            tiles = max(tiles, (start + min(r + HALF - 1, q_len - 1)) / LAT_TILE + 1);
+        }
+    }
+    if (tiles == 0) return;                             // (the whole workgroup)
     const int tid = threadIdx.x, wave = tid / NVA_WAVE, lane = tid % NVA_WAVE, col = lane & 15, g = lane >> 4;
-    const int row = row0 + wave;
+    const int row = HALF * (wave < HALF ? half_a : half_b) + wave % HALF;
     const bool token_ok = row < q_len;
     const int pos = token_ok ? start + row : -1;
-    const int64_t t = q_begin + (token_ok ? row : row0);
+    const int64_t t = q_begin + (token_ok ? row : 0);
     const int first = nva_first_key(pos, window, 0);
-    // the tiles that any token of the workgroup sees: the first token's window starts first
-    const int tile_0 = nva_first_key(start + row0, window, 0) / LAT_TILE;
-    const int tiles = (start + min(row0 + WAVES - 1, q_len - 1)) / LAT_TILE + 1;
     const int head = blockIdx.z * 16 + col;
     const bool head_ok = head < heads;
-    const int steps = (width + 31) / 32, blocks = rank / 16;
     const int32_t* table = block_tables + (int64_t)seq * table_stride;
     const int tiles_per_page = page_size / LAT_TILE;
-    const int k_pieces = 4 * width, v_pieces = 4 * rank;
 
+    // A row of keys lies in LDS in pieces of eight channels, piece p of key r at p ^ swizzle(r); a row of values in pieces of
+    // eight keys, piece p of channel c at p ^ (c / 2) % 4: eight lanes that read the same piece of eight rows meet no bank
+    // twice.
+    auto swizzle = [](int r) { return (r & 3) | (r >> 1 & 4); };
+    // (channels past a key's are read as zeros; rows of values past the latent's only reach results that nobody stores)
+    if (width < KROW)
+        for (int i = tid; i < 2 * LAT_TILE * (KROW / 8); i += THREADS) {
+            const int r = i / (KROW / 8), p = i % (KROW / 8);
+            if ((p ^ swizzle(r % LAT_TILE)) * 8 >= width) *reinterpret_cast<lat_bf16x8*>(&lat_s[r / LAT_TILE * BUFFER + r % LAT_TILE * KROW + p * 8]) = lat_bf16x8{};
+        }
     lat_bf16x8 qf[KS];
     const __bf16* qrow = q2 + t * q_stride + (int64_t)(head_ok ? head : 0) * width;
 #pragma unroll
     for (int c = 0; c < KS; ++c) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) qf[c][e] = (__bf16)0.f;
-        if (c < steps && head_ok && token_ok && 32 * c + 8 * g < width) qf[c] = *reinterpret_cast<const lat_bf16x8*>(qrow + 32 * c + 8 * g);
+        qf[c] = lat_bf16x8{};
+        if (head_ok && token_ok && 32 * c + 8 * g < width) qf[c] = *reinterpret_cast<const lat_bf16x8*>(qrow + 32 * c + 8 * g);
     }
     lat_f32x4 acc[CB];
 #pragma unroll
@@ -652,79 +684,80 @@ latent_attn_quad_kernel(const __bf16* __restrict__ q2, int64_t q_stride, __bf16*
     float m_run = with_sink ? sinks[head] : -INFINITY, l_run = with_sink ? 1.f : 0.f;
     const float log2e = 1.4426950408889634f;
 
-    lat_bf16x8 kreg[KP], vreg[VP];
-    bool no_page = false, no_page_next = false;
-    auto ask = [&](int tile) __attribute__((always_inline)) {       // a tile's keys and values, as they lie in the cache, into registers
-        const int kb = tile * LAT_TILE;
-        int page = table[kb / page_size];
-        no_page_next = page < 0;
-        if (no_page_next) {
-            if (error_flag && tid == 0) atomicOr(error_flag, 2);    // a visible key has no page
+    auto page_of = [&](int tile) { return table[min(tile, tiles - 1) * LAT_TILE / page_size]; };
+    // where this lane's pieces lie in a tile, in bytes (the same in every tile)
+    const int unit_0 = __builtin_amdgcn_readfirstlane(wave);
+    int k_from[KOWN];
+#pragma unroll
+    for (int i = 0; i < KOWN; ++i) {
+        const int p = (unit_0 + WAVES * i) * NVA_WAVE + lane, r = p / (KROW / 8), c = 8 * (p % (KROW / 8) ^ swizzle(r));
+        k_from[i] = r < LAT_TILE && c < width ? 2 * (r * width + c) : -1;
+    }
+    const int v_from = 64 * (lane / 4) + 16 * (lane % 4 ^ lane / 8 % 4);
+    const uint32_t lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lat_s;
+    auto ask = [&](int tile, int page, int buffer) __attribute__((always_inline)) {     // a tile's keys and values, from the cache into LDS
+        if (page < 0) {
+            if (error_flag && tid == 0) atomicOr(error_flag, 2);        // a visible key has no page
             page = 0;
         }
-        const int in_page = kb % page_size;
+        page = __builtin_amdgcn_readfirstlane(page);
+        const int in_page = __builtin_amdgcn_readfirstlane(tile * LAT_TILE % page_size);
         const __bf16* kbase = k_cache + ((int64_t)page * page_size + in_page) * width;
         const __bf16* vbase = v_cache + ((int64_t)page * tiles_per_page + in_page / LAT_TILE) * rank * LAT_TILE;
+        const uint32_t to = __builtin_amdgcn_readfirstlane((int)(lds + 2 * (buffer * BUFFER)));
 #pragma unroll
-        for (int i = 0; i < KP; ++i) {
-            const int p = tid + THREADS * i;
-            if (p < k_pieces) kreg[i] = *reinterpret_cast<const lat_bf16x8*>(kbase + (int64_t)p * 8);
+        for (int i = 0; i < KOWN; ++i) {
+            const int unit = unit_0 + WAVES * i;
+            if (k_from[i] >= 0) nva_load_to_lds(kbase, (uint32_t)k_from[i], to + 1024 * (uint32_t)unit);
         }
 #pragma unroll
-        for (int i = 0; i < VP; ++i) {
-            const int p = tid + THREADS * i;
-            if (p < v_pieces) vreg[i] = *reinterpret_cast<const lat_bf16x8*>(vbase + (int64_t)p * 8);
-        }
-    };
-    auto put = [&]() __attribute__((always_inline)) {
-        const int per_key = width / 8;
-#pragma unroll
-        for (int i = 0; i < KP; ++i) {
-            const int p = tid + THREADS * i;
-            if (p < k_pieces) *reinterpret_cast<lat_bf16x8*>(&k_s[(p / per_key) * KSTR + (p % per_key) * 8]) = kreg[i];
-        }
-#pragma unroll
-        for (int i = 0; i < VP; ++i) {
-            const int p = tid + THREADS * i;
-            if (p < v_pieces) {
-                // (rows of 36 elements: two 8-byte stores)
-                lat_bf16x4 lo, hi;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) lo[e] = vreg[i][e], hi[e] = vreg[i][4 + e];
-                __bf16* dst = &v_s[(p / 4) * VSTR + (p % 4) * 8];
-                *reinterpret_cast<lat_bf16x4*>(dst) = lo;
-                *reinterpret_cast<lat_bf16x4*>(dst + 4) = hi;
-            }
+        for (int i = 0; i < VOWN; ++i) {
+            const int unit = unit_0 + WAVES * i;
+            if (16 * unit < rank) nva_load_to_lds(vbase, (uint32_t)(1024 * unit + v_from), to + 2 * LAT_TILE * KROW + 1024 * (uint32_t)unit);
         }
     };
-    ask(tile_0);
+    int page = page_of(tile_0);
+    ask(tile_0, page, 0);
+    int page_next = page_of(tile_0 + 1);
+    const int k_row = 2 * (col & 12) + (col & 3);           // the keys of the first product's rows: this one and four on
+    const int k_at = k_row * KROW, k_at4 = k_at + 4 * KROW, k_swz = swizzle(k_row), v_at = col * LAT_TILE + 8 * (g ^ (col / 2 & 3));
     for (int tile = tile_0; tile < tiles; ++tile) {
-        const int kb = tile * LAT_TILE;
-        put();
-        no_page = no_page_next;
-        __syncthreads();
-        if (tile + 1 < tiles) ask(tile + 1);
+        const int kb = tile * LAT_TILE, buffer = (tile - tile_0) & 1;
+        const __bf16* const k_s = lat_s + buffer * BUFFER;
+        const __bf16* const v_s = k_s + LAT_TILE * KROW;
+        const bool no_page = page < 0;
+        page = page_next;
+        nva_wait_loads_but<0>();
+        nva_lds_barrier();                                  // this tile has arrived; the other buffer has been read
+        if (tile + 1 < tiles) ask(tile + 1, page, buffer ^ 1);
+        page_next = page_of(tile + 2);
         if (kb <= pos && kb + LAT_TILE > first) {           // (the same for the whole wave)
             lat_f32x4 sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
+            // reads of LDS run AHEAD steps before their products, in this order (left to itself the compiler keeps one ahead)
+            lat_bf16x8 ka[AHEAD + 1], kc[AHEAD + 1];
+            auto read_keys = [&](int c) __attribute__((always_inline)) {
+                ka[c % (AHEAD + 1)] = *reinterpret_cast<const lat_bf16x8*>(&k_s[k_at + 8 * ((4 * c + g) ^ k_swz)]);
+                kc[c % (AHEAD + 1)] = *reinterpret_cast<const lat_bf16x8*>(&k_s[k_at4 + 8 * ((4 * c + g) ^ k_swz)]);
+            };
+#pragma unroll
+            for (int c = 0; c < AHEAD; ++c) read_keys(c);
 #pragma unroll
             for (int c = 0; c < KS; ++c) {
-                if (c < steps) {
-                    lat_bf16x8 ka, kc;
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) ka[e] = kc[e] = (__bf16)0.f;
-                    if (32 * c + 8 * g < width) {
-                        ka = *reinterpret_cast<const lat_bf16x8*>(&k_s[col * KSTR + 32 * c + 8 * g]);
-                        kc = *reinterpret_cast<const lat_bf16x8*>(&k_s[(16 + col) * KSTR + 32 * c + 8 * g]);
-                    }
-                    sa = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka, qf[c], sa, 0, 0, 0);
-                    sb = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kc, qf[c], sb, 0, 0, 0);
-                }
+                if (c + AHEAD < KS) read_keys(c + AHEAD);
+                __builtin_amdgcn_sched_barrier(0);
+                sa = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[c % (AHEAD + 1)], qf[c], sa, 0, 0, 0);
+                sb = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kc[c % (AHEAD + 1)], qf[c], sb, 0, 0, 0);
             }
+            lat_bf16x8 vr[VAHEAD + 1];
+            auto read_values = [&](int b) __attribute__((always_inline)) { vr[b % (VAHEAD + 1)] = *reinterpret_cast<const lat_bf16x8*>(&v_s[v_at + 16 * b * LAT_TILE]); };
+#pragma unroll
+            for (int b = 0; b < VAHEAD; ++b) read_values(b);
+            __builtin_amdgcn_sched_barrier(0);
             float s[8];
             float m_new = m_run;
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                const int key = kb + (i < 4 ? 4 * g + i : 16 + 4 * g + i - 4);
+                const int key = kb + 8 * g + i;
                 const float raw = (i < 4 ? sa[i] : sb[i - 4]) * scale;
                 s[i] = key <= pos && key >= first && !no_page ? raw : -INFINITY;
                 m_new = fmaxf(m_new, s[i]);
@@ -743,36 +776,37 @@ latent_attn_quad_kernel(const __bf16* __restrict__ q2, int64_t q_stride, __bf16*
             const float alpha = __builtin_amdgcn_exp2f((fmaxf(m_run, -1e30f) - m_use) * log2e);
             l_run = l_run * alpha + psum;
             m_run = m_new;
-            const bool whole = kb + LAT_TILE - 1 <= pos && kb >= first && !no_page;
+            if (__any(alpha != 1.f)) {
 #pragma unroll
-            for (int b = 0; b < CB; ++b) {
-                if (b < blocks) {
-                    const lat_bf16x4 lo = *reinterpret_cast<const lat_bf16x4*>(&v_s[(16 * b + col) * VSTR + 4 * g]);
-                    const lat_bf16x4 hi = *reinterpret_cast<const lat_bf16x4*>(&v_s[(16 * b + col) * VSTR + 16 + 4 * g]);
-                    lat_bf16x8 vf;
+                for (int b = 0; b < CB; ++b) acc[b] *= alpha;
+            }
+            // (what the cache holds beyond the token's own key, or before its window, may be anything)
+            auto values = [&](auto whole) __attribute__((always_inline)) {
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) vf[e] = lo[e], vf[4 + e] = hi[e];
-                    if (!whole) {
+                for (int b = 0; b < CB; ++b) {
+                    if (b + VAHEAD < CB) read_values(b + VAHEAD);
+                    __builtin_amdgcn_sched_barrier(0);
+                    lat_bf16x8 vf = vr[b % (VAHEAD + 1)];
+                    if (!decltype(whole)::value) {
 #pragma unroll
                         for (int e = 0; e < 8; ++e) {
-                            const int key = kb + (e < 4 ? 4 * g + e : 16 + 4 * g + e - 4);
+                            const int key = kb + 8 * g + e;
                             if (no_page || key > pos || key < first) vf[e] = (__bf16)0.f;
                         }
                     }
-                    lat_f32x4 a = acc[b];
-                    a[0] *= alpha; a[1] *= alpha; a[2] *= alpha; a[3] *= alpha;
-                    acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf, a, 0, 0, 0);
+                    acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf, acc[b], 0, 0, 0);
                 }
-            }
+            };
+            if (kb + LAT_TILE - 1 <= pos && kb >= first && !no_page) values(std::true_type{});
+            else values(std::false_type{});
         }
-        __syncthreads();                                    // all have read the tile: the next may be stored
     }
     if (!head_ok || !token_ok) return;
     const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
     __bf16* orow = out + t * out_stride + (int64_t)head * rank;
 #pragma unroll
     for (int b = 0; b < CB; ++b)
-        if (b < blocks) {
+        if (16 * b < rank) {
             lat_bf16x4 v;
 #pragma unroll
             for (int i = 0; i < 4; ++i) v[i] = (__bf16)(acc[b][i] * inv);
@@ -881,26 +915,27 @@ NVA_EXPORT int nva_latent_attention_prefill_bf16(const void* q2, int64_t q_strid
         nva_fail("latent_attention_prefill: rows that are not aligned for vector access");
         return 1;
     }
-    const size_t lds = ((size_t)LAT_TILE * (rank + rot + 8) + (size_t)rank * (LAT_TILE + 4)) * sizeof(__bf16);
-    const int waves = rank <= 384 ? 8 : 4;       // tokens of a workgroup (what the registers of a SIMD hold two waves of)
-    dim3 grid((unsigned)(num_tiles * (32 / waves)), 1, (unsigned)((heads + 15) / 16));
-#define LAT_LAUNCH(MC, WV)                                                                                           \
+#define LAT_LAUNCH(MC, MR, WV)                                                                                       \
     do {                                                                                                             \
-        auto kernel = latent_attn_quad_kernel<MC, WV>;                                                                 \
+        auto kernel = latent_attn_rows_kernel<MC, MR, WV>;                                                             \
+        const size_t lds = 2 * ((size_t)LAT_TILE * (MC + MR + MC)) * sizeof(__bf16);        \
         static bool raised = false;                                                                                  \
         if (!raised && lds > 48 * 1024) {                                                                            \
-            if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024) != hipSuccess) \
+            if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) \
                 return nva_fail("latent_attention_prefill: cannot have %zu bytes of LDS", lds);                      \
             raised = true;                                                                                           \
         }                                                                                                            \
-        hipLaunchKernelGGL(kernel, grid, dim3(WV * NVA_WAVE), lds, stream, (const __bf16*)q2, q_stride, (__bf16*)out,    \
-                           out_stride, (const __bf16*)k_cache, (const __bf16*)v_cache, block_tables, table_stride,      \
-                           cu_seqlens_q, kv_lens, row_tiles, heads, rank, rot, page_size, scale, window, sinks, error_flag);    \
+        hipLaunchKernelGGL(kernel, dim3((unsigned)(num_tiles * (32 / WV)), 1, (unsigned)((heads + 15) / 16)), dim3(WV * NVA_WAVE), lds, \
+                           stream, (const __bf16*)q2, q_stride, (__bf16*)out, out_stride, (const __bf16*)k_cache,                   \
+                           (const __bf16*)v_cache, block_tables, table_stride, cu_seqlens_q, kv_lens, row_tiles, heads, rank, rot,   \
+                           page_size, scale, window, sinks, error_flag);                                             \
     } while (0)
-    if (rank <= 128) LAT_LAUNCH(128, 8);
-    else if (rank <= 256) LAT_LAUNCH(256, 8);
-    else if (rank <= 384) LAT_LAUNCH(384, 8);
-    else LAT_LAUNCH(512, 4);
+#define LAT_RANK(MC, WV) do { if (rot <= 64) LAT_LAUNCH(MC, 64, WV); else LAT_LAUNCH(MC, 128, WV); } while (0)
+    if (rank <= 128) LAT_RANK(128, 8);
+    else if (rank <= 256) LAT_RANK(256, 8);
+    else if (rank <= 384) LAT_RANK(384, 8);
+    else LAT_RANK(512, 4);
+#undef LAT_RANK
 #undef LAT_LAUNCH
     return nva_check_launch("latent_attention_prefill");
 }
