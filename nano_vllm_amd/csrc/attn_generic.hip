@@ -604,6 +604,166 @@ paged_attention_tiled_kernel(const T* __restrict__ q, int64_t q_stride, T* __res
     }
 }
 
+#if defined(NVA_F32)
+// The tiled kernel for keys and values of the same 64 or 128 channels, without chunks, where blocks of 64 keys lie within pages:
+// the same arithmetic again, bit for bit.  A block's keys and values are on their way into registers while the block before
+// is at work, and lie in LDS in pieces of four, piece p of a row r at p ^ r % 8 (a lane reads its key, or its channel, four at a
+// time, eight lanes meeting no bank twice).  The queries are the wave's own and the same in every lane: they come through the
+// scalar cache as operands of the products instead of through LDS, whose reads of one address cost as much as any, and leave
+// room for two workgroups a compute unit.  Weights of zero are looked for once a block: only where there are any is every
+// addition a choice.
+// Bound by the vector units: 128 products, 128 additions and 64 broadcasts of weights a lane, row and block, in the workgroups
+// with the most keys.  16 heads of 128, three portions of up to 600 tokens: 139 us, the kernel above 249.
+template <int D>
+__global__ void __launch_bounds__(ATT_TILED_WAVES * NVA_WAVE, 4)
+paged_attention_rows_kernel(const float* __restrict__ q, int64_t q_stride, float* __restrict__ out, int64_t out_stride,
+                            const float* __restrict__ k_cache, const float* __restrict__ v_cache,
+                            const int32_t* __restrict__ block_tables, int table_stride, const int32_t* __restrict__ cu_seqlens_q,
+                            const int32_t* __restrict__ kv_lens, const int32_t* __restrict__ tiles, int num_q_heads, int num_kv_heads,
+                            int page_size, float scale, float softcap, const float* __restrict__ sinks,
+                            const float* __restrict__ head_gate, int32_t* error_flag) {
+    constexpr int THREADS = ATT_TILED_WAVES * NVA_WAVE, ROWS = ATT_ROWS / ATT_TILED_WAVES, ACC = D / NVA_WAVE;
+    constexpr int PIECES = NVA_WAVE * D / 4 / THREADS;              // of a thread, of keys and of values
+    static_assert(ROWS == 4, "");
+    __shared__ __attribute__((aligned(16))) float k_s[NVA_WAVE * D], v_s[NVA_WAVE * D];     // [64 keys][D], [D][64 keys]
+    const int seq = tiles[2 * blockIdx.x], tile = tiles[2 * blockIdx.x + 1];
+    const int h = blockIdx.y;
+    const int kvh = h / (num_q_heads / num_kv_heads);
+    const int q_begin = cu_seqlens_q[seq];
+    const int q_len = cu_seqlens_q[seq + 1] - q_begin;
+    const int start = kv_lens[seq] - q_len;                          // position of the request's first query of this step
+    const int q0 = tile * ATT_ROWS;
+    const int rows = min(ATT_ROWS, q_len - q0);
+    const int last_pos = start + q0 + rows - 1;
+    const int32_t* table = block_tables + (int64_t)seq * table_stride;
+    const int tid = threadIdx.x, lane = tid % NVA_WAVE, wave = __builtin_amdgcn_readfirstlane(tid / NVA_WAVE);
+
+    // row t of the wave: wave + 8 t
+    float acc[ROWS][ACC], m_run[ROWS], l_run[ROWS];
+    int pos[ROWS], last = -1;
+    const float* qr[ROWS];
+#pragma unroll
+    for (int t = 0; t < ROWS; ++t) {
+        const int r = wave + ATT_TILED_WAVES * t;
+        pos[t] = r < rows ? start + q0 + r : -1;
+        last = max(last, pos[t]);
+        qr[t] = q + (int64_t)(q_begin + q0 + min(r, rows - 1)) * q_stride + (int64_t)h * D;
+#pragma unroll
+        for (int i = 0; i < ACC; ++i) acc[t][i] = 0.f;
+        m_run[t] = sinks ? sinks[h] : -INFINITY, l_run[t] = sinks ? 1.f : 0.f;
+    }
+    float4 kk0, kk1, kk2, kk3, vv0, vv1, vv2, vv3;                   // (64 keys lie side by side in either cache)
+    const int swz = 4 * (lane & 7);
+    const float* const kr = k_s + lane * D;
+    const float* const vr = v_s + lane * NVA_WAVE;
+    auto page_of = [&](int base) { return __builtin_amdgcn_readfirstlane(table[min(base, last_pos) / page_size]); };
+#define ATT_ASK(BASE, PAGE)                                                                                           \
+    do {                                                                                                              \
+        const int64_t block = (((int64_t)max(PAGE, 0) * num_kv_heads + kvh) * page_size + (BASE) % page_size) * D;         \
+        const float4* ka = reinterpret_cast<const float4*>(k_cache + block) + tid;                                       \
+        const float4* va = reinterpret_cast<const float4*>(v_cache + block) + tid;                                       \
+        kk0 = ka[0], vv0 = va[0], kk1 = ka[THREADS], vv1 = va[THREADS];                                                 \
+        if (PIECES == 4) kk2 = ka[2 * THREADS], vv2 = va[2 * THREADS], kk3 = ka[3 * THREADS], vv3 = va[3 * THREADS];        \
+    } while (0)
+    int page = page_of(0);
+    ATT_ASK(0, page);
+    int page_next = page_of(NVA_WAVE);
+    for (int base = 0; base <= last_pos; base += NVA_WAVE) {
+        __syncthreads();                                             // the chunk before is done with
+        auto put = [&](int u, float4 k4, float4 v4) __attribute__((always_inline)) {
+            const int i = tid + THREADS * u, key = i / (D / 4), pc = i % (D / 4);
+            *reinterpret_cast<float4*>(&k_s[key * D + 4 * (pc ^ (key & 7))]) = k4;
+            const int d = i / 8 % D, vp = i / (8 * D) * 8 + i % 8;   // values: tiles of [D][32 keys]
+            *reinterpret_cast<float4*>(&v_s[d * NVA_WAVE + 4 * (vp ^ (d & 7))]) = v4;
+        };
+        put(0, kk0, vv0);
+        put(1, kk1, vv1);
+        if (PIECES == 4) put(2, kk2, vv2), put(3, kk3, vv3);
+        __syncthreads();
+        const bool key_ok = page >= 0;
+        if (!key_ok && error_flag && tid == 0) atomicOr(error_flag, 2);           // a visible key has no page
+        page = page_next;
+        if (base + NVA_WAVE <= last_pos) ATT_ASK(base + NVA_WAVE, page);
+        page_next = page_of(base + 2 * NVA_WAVE);
+        if (base > last) continue;                                   // (the same for the whole wave)
+        float dot[ROWS] = {0.f, 0.f, 0.f, 0.f};
+        // (a loop, or the compiler would ask for all the wave's queries before the first product)
+#pragma unroll 1
+        for (int d = 0; d < D; d += 8) {
+            float qe[ROWS][8];
+#pragma unroll
+            for (int t = 0; t < ROWS; ++t)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) qe[t][e] = qr[t][d + e];
+            const float4 k4[2] = {*reinterpret_cast<const float4*>(kr + (d & 28 ^ swz) + (d & ~31)), *reinterpret_cast<const float4*>(kr + (d + 4 & 28 ^ swz) + (d & ~31))};
+#pragma unroll
+            for (int half = 0; half < 2; ++half) {
+                const float ke[4] = {k4[half].x, k4[half].y, k4[half].z, k4[half].w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int t = 0; t < ROWS; ++t) dot[t] += qe[t][4 * half + e] * ke[e];
+            }
+        }
+        float p[ROWS];
+        bool full = true;
+#pragma unroll
+        for (int t = 0; t < ROWS; ++t) {
+            float s = dot[t] * scale;
+            if (softcap > 0.f) s = softcap * tanhf(s / softcap);
+            if (!(base + lane <= pos[t] && key_ok)) s = -INFINITY;
+            const float m_new = fmaxf(m_run[t], wave_max(s));
+            p[t] = (s == -INFINITY) ? 0.f : nva_exp(s - m_new);
+            const float correction = (m_run[t] == -INFINITY) ? 0.f : nva_exp(m_run[t] - m_new);
+            l_run[t] = l_run[t] * correction + wave_sum(p[t]);
+            m_run[t] = m_new;
+            full = full && p[t] != 0.f;
+#pragma unroll
+            for (int i = 0; i < ACC; ++i) acc[t][i] *= correction;
+        }
+        // channel d = lane + 64 i adds its keys in ascending order; a key of weight zero (masked, or beyond the row's position)
+        // adds nothing, whatever V holds
+        auto add_keys = [&](int vp, int at, auto choose) __attribute__((always_inline)) {
+            float ve[ACC][4];
+#pragma unroll
+            for (int i = 0; i < ACC; ++i) {
+                const float4 v4 = *reinterpret_cast<const float4*>(vr + NVA_WAVE * NVA_WAVE * i + at);
+                ve[i][0] = v4.x, ve[i][1] = v4.y, ve[i][2] = v4.z, ve[i][3] = v4.w;
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int t = 0; t < ROWS; ++t) {
+                    const float pj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p[t]), 4 * vp + u));
+#pragma unroll
+                    for (int i = 0; i < ACC; ++i) {
+                        const float with = acc[t][i] + pj * ve[i][u];
+                        acc[t][i] = !decltype(choose)::value || pj != 0.f ? with : acc[t][i];
+                    }
+                }
+        };
+        if (__all(full)) {
+#pragma unroll 2
+            for (int vp = 0; vp < NVA_WAVE / 4; ++vp) add_keys(vp, 4 * vp ^ swz, Count<0>());
+        } else {
+#pragma unroll 1
+            for (int vp = 0; vp < min(NVA_WAVE / 4, (last - base) / 4 + 1); ++vp) add_keys(vp, 4 * vp ^ swz, Count<1>());
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < ROWS; ++t) {
+        const int r = wave + ATT_TILED_WAVES * t;
+        if (r >= rows) continue;
+        float inv = l_run[t] > 0.f ? 1.f / l_run[t] : 0.f;
+        if (head_gate) inv *= head_gate[(int64_t)(q_begin + q0 + r) * num_q_heads + h];
+        float* orow = out + (int64_t)(q_begin + q0 + r) * out_stride + (int64_t)h * D;
+#pragma unroll
+        for (int i = 0; i < ACC; ++i) orow[lane + i * NVA_WAVE] = acc[t][i] * inv;
+    }
+}
+#undef ATT_ASK
+#endif
+
 // The same attention for portions of prompts, 32 rows of a request to a workgroup: tiles is int32
 // [num_tiles][2] = (request, row tile of 32 queries), requests described by cu_seqlens_q and kv_lens as
 // for the matrix-core kernel.  No window (chunks: yes), head sizes up to 128; returns 1 for what it does not take.
@@ -623,6 +783,16 @@ NVA_EXPORT int NVA_NAME(nva_paged_attention_tiled)(
     if (num_q_heads <= 0 || num_kv_heads <= 0 || num_q_heads % num_kv_heads || num_q_heads > 65535)
         return nva_fail("paged_attention_tiled: %d query heads do not divide into %d kv heads", num_q_heads, num_kv_heads);
     if (page_size <= 0 || table_stride <= 0) return nva_fail("paged_attention_tiled: bad page size or table width");
+#if defined(NVA_F32)
+    if (head_dim == v_dim && (head_dim == 64 || head_dim == 128) && chunk == 0 && page_size % NVA_WAVE == 0 && nva_aligned(k_cache, 16) &&
+        nva_aligned(v_cache, 16)) {
+        auto rows = head_dim == 64 ? paged_attention_rows_kernel<64> : paged_attention_rows_kernel<128>;
+        hipLaunchKernelGGL(rows, dim3((unsigned)num_tiles, (unsigned)num_q_heads), dim3(ATT_TILED_WAVES * NVA_WAVE), 0, stream, (const float*)q,
+                           q_stride, (float*)out, out_stride, (const float*)k_cache, (const float*)v_cache, block_tables, table_stride,
+                           cu_seqlens_q, kv_lens, tiles, num_q_heads, num_kv_heads, page_size, scale, softcap, sinks, head_gate, error_flag);
+        return nva_check_launch("paged_attention_tiled");
+    }
+#endif
     const size_t lds = att_tiled_lds(head_dim, v_dim);
     auto kernel = paged_attention_tiled_kernel<elem_t>;
     static bool raised = false;              // the kernel's LDS limit, lifted once to what the largest head size needs
