@@ -63,3 +63,40 @@ def test_rows_that_are_not_aligned():
     got = k.moe_experts(wide.to(DEV)[:, 1:129], ids.to(DEV), weights.to(DEV), up.to(DEV), down.to(DEV), 3, "silu", gated=True)
     want = _want(x, ids, weights, up, down, 3, True)
     assert float((got.double().cpu() - want).abs().max()) <= 2 ** -7 * float(want.abs().max())
+
+
+@pytest.mark.parametrize("routing", ["sigmoid_groups", "softmax_top", "softmax_choice", "softmax_scores"])
+@pytest.mark.parametrize("experts,groups,keep,top", [(64, 1, 1, 8), (64, 8, 3, 24), (32, 4, 2, 8), (63, 21, 5, 3), (6, 6, 2, 2), (1, 1, 1, 1), (64, 64, 64, 64)])
+def test_routing_with_an_expert_a_lane(routing, experts, groups, keep, top):
+    """Up to 64 experts and more run kernels of their own: groups of experts that nobody chooses beside them change no bit.
+    Many scores are equal (the lower number goes first)."""
+    from nano_vllm_amd.kernels import HipKernels
+    k = HipKernels(DEV, torch.bfloat16, quiet=True)
+    g = torch.Generator().manual_seed(experts + top)
+    logits = (torch.randn((37, experts), generator=g) * 4).round() / 2
+    bias = (torch.randn(experts, generator=g) * 2).round() / 8 if routing in ("softmax_top", "softmax_choice") else None
+    if routing == "softmax_top":
+        groups = keep = 1
+    per = experts // groups
+    more = (64 // per + 1) * per
+    wide = torch.cat((logits, torch.full((37, more), float("-inf"))), 1)
+    wide_bias = None if bias is None else torch.cat((bias, torch.full((more,), -9.0)))
+    dev = lambda t: None if t is None else t.to(DEV)
+    one = k.moe_route(dev(logits), top, groups, keep, 1.7, routing=routing, bias=dev(bias))
+    two = k.moe_route(dev(wide), top, groups + more // per, keep, 1.7, routing=routing, bias=dev(wide_bias)) if routing != "softmax_top" else \
+        k.moe_route(dev(wide), top, 1, 1, 1.7, routing=routing, bias=dev(wide_bias))
+    assert torch.equal(one[0], two[0]) and torch.equal(one[1], two[1])
+    assert int(one[0].max()) < experts and all(len(set(r)) == top for r in one[0].tolist())
+
+
+@pytest.mark.parametrize("tokens", [2047, 2048, 2049])
+def test_more_pairs_than_the_plan_keeps(tokens):
+    """8 choices of a token: 16384 pairs are what the plan's workgroup keeps in registers."""
+    from nano_vllm_amd.kernels import HipKernels
+    k = HipKernels(DEV, torch.bfloat16, quiet=True)
+    g = torch.Generator().manual_seed(tokens)
+    x, up, down = (torch.randn(s, generator=g).bfloat16().to(DEV) for s in ((tokens, 64), (10 * 64, 64), (10 * 64, 64)))
+    ids = torch.rand((tokens, 12), generator=g).topk(8, 1)[1].int().to(DEV)         # (10 and 11: identities)
+    weights = torch.rand((tokens, 8), generator=g).to(DEV)
+    run = lambda a, b: k.moe_experts(x[a:b], ids[a:b].contiguous(), weights[a:b].contiguous(), up, down, 10)
+    assert torch.equal(run(0, tokens), torch.cat((run(0, 1000), run(1000, tokens))))
