@@ -613,8 +613,8 @@ paged_attention_tiled_kernel(const T* __restrict__ q, int64_t q_stride, T* __res
 // room for two workgroups a compute unit.  Weights of zero are looked for once a block: only where there are any is every
 // addition a choice.
 // Bound by the vector units: 128 products, 128 additions and 64 broadcasts of weights a lane, row and block, in the workgroups
-// with the most keys.  16 heads of 128, three portions of up to 600 tokens: 139 us, the kernel above 249.
-template <int D>
+// with the most keys.  16 heads of 128, three portions of up to 600 tokens: 125 us, the kernel above 249.
+template <int D, int ROWS>
 __global__ void __launch_bounds__(ATT_TILED_WAVES * NVA_WAVE, 4)
 paged_attention_rows_kernel(const float* __restrict__ q, int64_t q_stride, float* __restrict__ out, int64_t out_stride,
                             const float* __restrict__ k_cache, const float* __restrict__ v_cache,
@@ -622,9 +622,8 @@ paged_attention_rows_kernel(const float* __restrict__ q, int64_t q_stride, float
                             const int32_t* __restrict__ kv_lens, const int32_t* __restrict__ tiles, int num_q_heads, int num_kv_heads,
                             int page_size, float scale, float softcap, const float* __restrict__ sinks,
                             const float* __restrict__ head_gate, int32_t* error_flag) {
-    constexpr int THREADS = ATT_TILED_WAVES * NVA_WAVE, ROWS = ATT_ROWS / ATT_TILED_WAVES, ACC = D / NVA_WAVE;
+    constexpr int THREADS = ATT_TILED_WAVES * NVA_WAVE, ACC = D / NVA_WAVE;
     constexpr int PIECES = NVA_WAVE * D / 4 / THREADS;              // of a thread, of keys and of values
-    static_assert(ROWS == 4, "");
     __shared__ __attribute__((aligned(16))) float k_s[NVA_WAVE * D], v_s[NVA_WAVE * D];     // [64 keys][D], [D][64 keys]
     const int seq = tiles[2 * blockIdx.x], tile = tiles[2 * blockIdx.x + 1];
     const int h = blockIdx.y;
@@ -632,8 +631,9 @@ paged_attention_rows_kernel(const float* __restrict__ q, int64_t q_stride, float
     const int q_begin = cu_seqlens_q[seq];
     const int q_len = cu_seqlens_q[seq + 1] - q_begin;
     const int start = kv_lens[seq] - q_len;                          // position of the request's first query of this step
-    const int q0 = tile * ATT_ROWS;
-    const int rows = min(ATT_ROWS, q_len - q0);
+    const int q0 = tile * ATT_ROWS + ATT_TILED_WAVES * ROWS * blockIdx.z;
+    const int rows = min(ATT_TILED_WAVES * ROWS, q_len - q0);
+    if (rows <= 0) return;                                           // (the whole workgroup)
     const int last_pos = start + q0 + rows - 1;
     const int32_t* table = block_tables + (int64_t)seq * table_stride;
     const int tid = threadIdx.x, lane = tid % NVA_WAVE, wave = __builtin_amdgcn_readfirstlane(tid / NVA_WAVE);
@@ -686,7 +686,9 @@ paged_attention_rows_kernel(const float* __restrict__ q, int64_t q_stride, float
         if (base + NVA_WAVE <= last_pos) ATT_ASK(base + NVA_WAVE, page);
         page_next = page_of(base + 2 * NVA_WAVE);
         if (base > last) continue;                                   // (the same for the whole wave)
-        float dot[ROWS] = {0.f, 0.f, 0.f, 0.f};
+        float dot[ROWS];
+#pragma unroll
+        for (int t = 0; t < ROWS; ++t) dot[t] = 0.f;
         // (a loop, or the compiler would ask for all the wave's queries before the first product)
 #pragma unroll 1
         for (int d = 0; d < D; d += 8) {
@@ -786,8 +788,13 @@ NVA_EXPORT int NVA_NAME(nva_paged_attention_tiled)(
 #if defined(NVA_F32)
     if (head_dim == v_dim && (head_dim == 64 || head_dim == 128) && chunk == 0 && page_size % NVA_WAVE == 0 && nva_aligned(k_cache, 16) &&
         nva_aligned(v_cache, 16)) {
-        auto rows = head_dim == 64 ? paged_attention_rows_kernel<64> : paged_attention_rows_kernel<128>;
-        hipLaunchKernelGGL(rows, dim3((unsigned)num_tiles, (unsigned)num_q_heads), dim3(ATT_TILED_WAVES * NVA_WAVE), 0, stream, (const float*)q,
+        // Four rows a wave, or two where that leaves fewer than four workgroups a compute unit: the last tiles of a prompt have
+        // the most keys, and the step waits for them.  (480 tiles and heads of three prompts 139 and 125 us a layer; 2048 of one
+        // of 2048 tokens, four layers with their products, 41.97 and 42.42 ms.)
+        const bool few = num_tiles * num_q_heads < 1024;
+        auto rows = head_dim == 64 ? (few ? paged_attention_rows_kernel<64, 2> : paged_attention_rows_kernel<64, 4>)
+                                   : (few ? paged_attention_rows_kernel<128, 2> : paged_attention_rows_kernel<128, 4>);
+        hipLaunchKernelGGL(rows, dim3((unsigned)num_tiles, (unsigned)num_q_heads, few ? 2 : 1), dim3(ATT_TILED_WAVES * NVA_WAVE), 0, stream, (const float*)q,
                            q_stride, (float*)out, out_stride, (const float*)k_cache, (const float*)v_cache, block_tables, table_stride,
                            cu_seqlens_q, kv_lens, tiles, num_q_heads, num_kv_heads, page_size, scale, softcap, sinks, head_gate, error_flag);
         return nva_check_launch("paged_attention_tiled");

@@ -12,6 +12,7 @@ import torch
     (4, 2, 64, 64, [2, 31, 32, 33, 63, 64, 65, 129], [2, 31, 32, 33, 63, 64, 65, 129]),
     (3, 3, 128, 192, [64, 66, 128, 200, 500], [1, 2, 32, 33, 65]),
     (6, 1, 128, 256, [300, 97], [40, 97]),
+    (128, 128, 64, 64, [250, 33], [250, 33]),                # two rows a wave, and (above 1024 tiles and heads) four
 ])
 def test_portions_give_the_bits_of_one_wave_per_token(hq, hkv, D, page, lens, q_lens, scale, extras):
     from nano_vllm_amd.kernels import HipKernels
